@@ -152,6 +152,13 @@ size_t pmoe_moe_workspace(const pmoe_geom* g, int n, int k, int shared,
  * that reason about tile edges. */
 int pmoe_prefill_tile_rows(int n, int kk, int n_experts);
 
+/* 1 when the experts of n tokens with kk columns (shared: the last is a
+ * shared expert's) run as streamed 16-column tiles: between the decode GEMV
+ * (few rows an expert) and the prefill GEMMs (more than 32 rows an expert on
+ * average); PMOE_STREAM=1 / 0 pins it where the shape is covered.  No
+ * reference counterpart. */
+int pmoe_stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int shared);
+
 /* A MoE workspace starts with a 1,352,960-byte synchronisation header (grid
  * barrier counters, launch epoch and per-block flags of the one-launch
  * decode layer; launch and tile counters, tagged logit and h words and the

@@ -495,6 +495,16 @@ int decode_route(const GemvArgs& gu, const RouteDev& rt, int32_t* inds_out, floa
   PMOE_REQUIRE(ri.d % 8 == 0, "router_logits: hidden must be a multiple of 8");
   RouteRecord* rec = static_cast<RouteRecord*>(record);
   const int epl = (rt.e + 63) / 64;
+  if (rt.n > 1) {
+#define PMOE_EPL(EP) \
+  if (epl <= EP) return launch_router<EP>(ri, rt, rec, gu, inds_out, w_out, st);
+    PMOE_EPL(2)
+    PMOE_EPL(4)
+    PMOE_EPL(8)
+    PMOE_EPL(16)
+#undef PMOE_EPL
+    return fail(PMOE_EINVAL, "decode: too many experts");
+  }
   const int n = rt.n, n_w = rt.e;
   const int e = n_w + (ri.w_extra ? 1 : 0);
   RouteTail t{rt, rec, gu.table, gu.n_experts, gu.shared_slot, inds_out, w_out, ri.arrive};
@@ -521,6 +531,15 @@ int decode_route(const GemvArgs& gu, const RouteDev& rt, int32_t* inds_out, floa
   else
     return fail(PMOE_EINVAL, "decode: too many experts");
   PMOE_LAUNCH_CHECK("router_route_kernel");
+  return PMOE_OK;
+}
+
+int decode_combine(const float* y, const void* record, int n, int kk, int d, uint16_t* out,
+                   hipStream_t st) {
+  ProfScope prof_scope(K_COMBINE, st);
+  combine_y_kernel<<<dim3((d + 255) / 256, n), 256, 0, st>>>(
+      y, static_cast<const RouteRecord*>(record), kk, d, out);
+  PMOE_LAUNCH_CHECK("combine_y_kernel");
   return PMOE_OK;
 }
 

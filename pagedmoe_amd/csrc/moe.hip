@@ -188,6 +188,40 @@ int check_route_cfg(const pmoe_route_cfg* rc) {
   return PMOE_OK;
 }
 
+// Whether the experts of n tokens with kk columns run as streamed MFMA tiles
+// (stream.hip) rather than as the decode GEMV or the prefill GEMMs.  Measured
+// us a layer, GEMV or prefill form / streamed, on either side of each line:
+//   upper end, 32 rows an expert on average (the 32-row prefill tiles'
+//     range): Qwen3-235B shapes 512 tokens 607 / 490, 700 tokens 538 / 594
+//     (128-row tiles); Qwen3-Next shapes 1400 tokens 498 / 477.  Reductions
+//     above 4096 hold 16 rows a pass, not 32, and stop where the prefill GEMMs
+//     begin (DeepSeek-V3 shapes 600 tokens 25763 / 2734, 1000 tokens
+//     3183 / 3757).  Layers of hidden < 2048 keep the prefill GEMMs there,
+//     whose two tile heights give the same bits.
+//   lower end, where the GEMV's re-use of a weight row for the few rows of an
+//     expert runs out: 0.75 rows an expert for 4-bit (Qwen3-235B shapes 8
+//     tokens 129 / 149, 12 tokens 179 / 175, 20 tokens 273 / 226), 0.5 for
+//     6-bit (Qwen3-Next shapes 16 tokens 125 / 161, 24 tokens 233 / 169), 16
+//     rows for reductions above 4096 (DeepSeek-V3 shapes 2 tokens 134 / 122,
+//     8 tokens 438 / 316); and 128 MiB of GEMV reads (rows x expert bytes), so
+//     that the extra launches pay (hidden 1024, 32 experts: 24 tokens 46 / 50,
+//     40 tokens 61 / 54).
+// PMOE_STREAM=1 / 0 pins the form where it covers the shape (read per call, so
+// the two can be compared).
+bool stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int n_ids) {
+  if (!stream_covers(g)) return false;
+  const char* v = getenv("PMOE_STREAM");
+  if (v && (v[0] == '0' || v[0] == '1')) return v[0] == '1';
+  const long rows = long(n) * kk;
+  const bool wide = g->hidden > 4096 || g->inter > 4096;
+  if (prefill_wanted(g, n, kk, n_ids) &&
+      (wide || g->hidden < 2048 || getenv("PMOE_PREFILL_SMALL")))
+    return false;
+  if (rows > 32L * n_experts || rows * g->expert_bytes < (128L << 20)) return false;
+  if (wide) return rows >= 16;
+  return g->bits == 4 ? 4 * rows >= 3L * n_experts : 2 * rows >= n_experts;
+}
+
 // Dispatch + the three projections (+ SwiGLU) for rows = n*kk flat rows.
 // y receives [rows, hidden] (f32 when y_f32, else bf16).
 int run_experts(const pmoe_geom* g, const uint8_t* slab, const int32_t* table, int n_experts,
@@ -195,13 +229,16 @@ int run_experts(const pmoe_geom* g, const uint8_t* slab, const int32_t* table, i
                 int max_rows_per_expert, const MoeWs& w, void* y, int y_f32, hipStream_t st) {
   const int rows = n * kk;
   const int n_ids = n_experts + (kk > k ? 1 : 0);
-  const bool prefill = prefill_wanted(g, n, kk, n_ids);
-  const int tm = prefill ? prefill_tile_rows(n, kk, n_experts) : 0;
+  const bool stream = stream_wanted(g, n, kk, n_experts, n_ids);
+  const bool prefill = !stream && prefill_wanted(g, n, kk, n_ids);
+  const int tm = stream ? stream_tile_rows() : prefill ? prefill_tile_rows(n, kk, n_experts) : 0;
   // the tile list carries the slots of this table
   int rc = dispatch_ext(inds, rows, k, kk, n_ids, w.order, w.counts, w.offsets, w.inv, w.active,
                         w.n_active, tm, w.tiles, w.n_tiles, table, shared_slot, w.dws,
                         w.dws_bytes, st);
   if (rc) return rc;
+  if (stream)
+    return stream_experts(g, slab, x, n, kk, w.order, w.tiles, w.n_tiles, w.h, y, y_f32, st);
   if (prefill)
     return prefill_experts(g, slab, x, n, kk, w.order, w.tiles, w.n_tiles, tm,
                            std::min(rows / tm + n_ids + 1, w.max_tiles), w.h, y, y_f32, st);
@@ -332,6 +369,15 @@ int decode_block(const pmoe_geom* g, const pmoe_route_cfg* rc, const uint8_t* sl
                                 out, w.sync, st);
     if (r2 != kDecodeFusedDeclined) return r2;
   }
+  if (n > 1 && !getenv("PMOE_DECODE_FUSED") && stream_wanted(g, n, kk, e, e + shared)) {
+    // (a pinned decode form compares the GEMV paths) the router launch (routing in its last block), the dispatch of its
+    // picks, the streamed experts into fp32 per-slot rows, the combine
+    int r = decode_route(gu, rt, inds_out, w_out, w.record, ri, st);
+    if (r) return r;
+    r = run_experts(g, slab, table, e, shared_slot, x, inds_out, n, k, kk, n, w, w.y, 1, st);
+    if (r) return r;
+    return decode_combine(w.y, w.record, n, kk, g->hidden, out, st);
+  }
   dn.out = w.y;  // fp32 per-slot outputs when the down runs expert-split
   return decode_routed(gu, dn, rt, g->bits, inds_out, w_out, out, w.record, ri, st);
 }
@@ -388,6 +434,11 @@ int experts_and_combine(const pmoe_geom* g, const uint8_t* slab, const int32_t* 
 }  // namespace pmoe
 
 using pmoe::MoeWs;
+
+extern "C" int pmoe_stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int shared) {
+  if (!g || n <= 0 || kk <= 0 || n_experts <= 0) return 0;
+  return pmoe::stream_wanted(g, n, kk, n_experts, n_experts + (shared ? 1 : 0)) ? 1 : 0;
+}
 
 extern "C" size_t pmoe_moe_workspace(const pmoe_geom* g, int n, int k, int shared,
                                      int n_experts) {

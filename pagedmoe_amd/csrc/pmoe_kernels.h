@@ -93,6 +93,11 @@ size_t decode_record_bytes();
 int decode_route(const GemvArgs& gu, const RouteDev& rt, int32_t* inds_out, float* w_out,
                  void* record, const RouterIn& ri, hipStream_t st);
 
+// out[n, o] = sum over columns c of the record's weight times y[n*kk + c, o],
+// in c order (y fp32, [n*kk, d]).
+int decode_combine(const float* y, const void* record, int n, int kk, int d, uint16_t* out,
+                   hipStream_t st);
+
 // Grid-barrier state of the fused decode launch: the first kDecodeSyncBytes
 // of the MoE workspace, zero before the first call.  Blocks arrive in groups
 // of kDecodeGroup: group g's counter for barrier i (its own 128-byte line at
@@ -193,6 +198,15 @@ int route_softmax(const float* logits, int n, int e, int k, int norm, int32_t* i
 int route_sigmoid(const float* logits, const float* bias, int n, int e, int n_group,
                   int topk_group, int k, int norm, float scale, int32_t* inds, float* weights,
                   hipStream_t st);
+
+// Experts of few rows each over the dispatch's tiles of stream_tile_rows()
+// rows (stream.hip): gate/up into h, down into y [rows, hidden] (fp32 when
+// y_f32, else bf16).
+bool stream_covers(const pmoe_geom* g);
+int stream_tile_rows();
+int stream_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
+                   const int32_t* order, const int4* tiles, const int32_t* n_tiles, uint16_t* h,
+                   void* y, int y_f32, hipStream_t st);
 
 // Dispatch (dispatch.hip).  Flat row r reads id inds[(r / kk) * k_routed +
 // r % kk] when r % kk < k_routed and the shared pseudo-id n_routed otherwise;
