@@ -38,31 +38,47 @@ __device__ __forceinline__ int load_id(const IdSrc& src, int r) {
   return (e >= 0 && e < src.n_routed) ? e : -1;
 }
 
-// Rank of each thread's row among the earlier rows of its block with the same
-// expert, and the block's rows per expert.  s_e[] holds the block's ids (-1:
-// none, also past the rows; 16-byte aligned), s_wc[e * NW + w] receives wave
-// w's rows of expert e as a byte (at most 64) and must be zero.  A lane
-// compares its id with its wave's 64 (16 broadcast reads), and the waves'
-// counts of an expert are read as one word or quad.  (One scan over all
-// earlier rows, up to 1,023 dependent steps, made an 800-row dispatch 16.0 us
-// (rocprof) against 8.1 now, and the 256-row counting blocks 6.2 against 4.9.)
-template <int NW>
-__device__ __forceinline__ int block_rank(int my_e, const int* s_e, uint8_t* s_wc) {
-  static_assert(NW == 4 || NW == 16, "4 or 16 waves");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int4* v = reinterpret_cast<const int4*>(s_e + wave * 64);
-  int rank = 0, in_wave = 0;
+// Rank of the lane's id among the earlier lanes of its wave, and how often the
+// wave's `rows` ids (s_e, 16-byte aligned) hold it.
+__device__ __forceinline__ int wave_rank(int my_e, int rows, const int* s_e, int& in_wave) {
+  const int lane = threadIdx.x & 63;
+  const int4* v = reinterpret_cast<const int4*>(s_e);
+  int rank = 0;
+  in_wave = 0;
+  // 16 ids a trip, only as many as the wave has rows
+  for (int i0 = 0; i0 < 16 && 4 * i0 < rows; i0 += 4) {
+    int4 q[4];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int4 q = v[i];
-    const int ids[4] = {q.x, q.y, q.z, q.w};
+    for (int i = 0; i < 4; ++i) q[i] = v[i0 + i];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int same = ids[j] == my_e ? 1 : 0;
-      in_wave += same;
-      rank += 4 * i + j < lane ? same : 0;
+    for (int i = 0; i < 4; ++i) {
+      const int ids[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int same = ids[j] == my_e ? 1 : 0;
+        in_wave += same;
+        rank += 4 * (i0 + i) + j < lane ? same : 0;
+      }
     }
   }
+  return rank;
+}
+
+// Rank of each thread's row among the earlier rows of its block with the same
+// expert, and the block's rows per expert (rows: how many the block has).
+// s_e[] holds the block's ids (-1: none, also past the rows; 16-byte aligned), s_wc[e * NW + w] receives wave
+// w's rows of expert e as a byte (at most 64) and must be zero.  A lane
+// compares its id with its wave's (wave_rank: broadcast reads), and the waves'
+// counts of an expert are read as one word or quad.  (One scan over all
+// earlier rows, up to 1,023 dependent steps, made an 800-row dispatch 16.0 us
+// (rocprof) against 8.1 now, and the 256-row counting blocks 6.2 against 4.9;
+// up to 64 rows one wave's ranks are all there is.)
+template <int NW>
+__device__ __forceinline__ int block_rank(int my_e, int rows, const int* s_e, uint8_t* s_wc) {
+  static_assert(NW == 4 || NW == 16, "4 or 16 waves");
+  const int wave = threadIdx.x >> 6;
+  int in_wave;
+  int rank = wave_rank(my_e, rows - wave * 64, s_e + wave * 64, in_wave);
   if (my_e >= 0 && rank == in_wave - 1) s_wc[my_e * NW + wave] = uint8_t(in_wave);
   __syncthreads();
   if (my_e >= 0) {
@@ -192,12 +208,23 @@ __global__ __launch_bounds__(1024) void dispatch_small_kernel(
   __shared__ int s_off[kMaxExperts];
   __shared__ int s_tmp[48];
   const int tid = threadIdx.x;
-  reinterpret_cast<uint4*>(s_wc)[tid] = make_uint4(0, 0, 0, 0);
+  const bool one_wave = rows <= 64;  // no counts to add up over waves
+  if (one_wave)
+    s_cnt[tid] = 0;
+  else
+    reinterpret_cast<uint4*>(s_wc)[tid] = make_uint4(0, 0, 0, 0);
   const int my_e = tid < rows ? load_id(src, tid) : -1;
   s_e[tid] = my_e;
   __syncthreads();
-  const int rank = block_rank<16>(my_e, s_e, s_wc);
-  if (tid < n_experts) s_cnt[tid] = block_count<16>(s_wc, tid);
+  int rank = 0;
+  if (one_wave) {
+    int in_wave;
+    rank = tid < 64 ? wave_rank(my_e, rows, s_e, in_wave) : 0;
+    if (my_e >= 0 && rank == in_wave - 1) s_cnt[my_e] = in_wave;
+  } else {
+    rank = block_rank<16>(my_e, rows, s_e, s_wc);
+    if (tid < n_experts) s_cnt[tid] = block_count<16>(s_wc, tid);
+  }
   __syncthreads();
   finish_scan(s_cnt, n_experts, counts, offsets, active, n_active, ts, s_off, s_tmp);
   if (my_e >= 0) {
@@ -221,7 +248,7 @@ __global__ __launch_bounds__(kChunk) void dispatch_count_kernel(
   const int my_e = row < rows ? load_id(src, row) : -1;
   s_e[tid] = my_e;
   __syncthreads();
-  const int rank = block_rank<4>(my_e, s_e, s_wc);
+  const int rank = block_rank<4>(my_e, rows - int(blockIdx.x) * kChunk, s_e, s_wc);
   if (my_e >= 0) rank_out[row] = rank;
   for (int e = tid; e < n_experts; e += kChunk)
     hist[size_t(blockIdx.x) * n_experts + e] = block_count<4>(s_wc, e);
