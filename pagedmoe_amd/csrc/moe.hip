@@ -193,15 +193,17 @@ int check_route_cfg(const pmoe_route_cfg* rc) {
 // us a layer, GEMV or prefill form / streamed, on either side of each line:
 //   upper end, 32 rows an expert on average (the 32-row prefill tiles'
 //     range): Qwen3-235B shapes 512 tokens 607 / 490, 700 tokens 538 / 594
-//     (128-row tiles); Qwen3-Next shapes 1400 tokens 498 / 477.  Reductions
+//     (128-row tiles); Qwen3-Next shapes 1000 tokens 422 / 399,
+//     1400 tokens 493 / 466.  Reductions
 //     above 4096 hold 16 rows a pass, not 32, and stop where the prefill GEMMs
 //     begin (DeepSeek-V3 shapes 600 tokens 25763 / 2734, 1000 tokens
 //     3183 / 3757).  Layers of hidden < 2048 keep the prefill GEMMs there,
 //     whose two tile heights give the same bits.
 //   lower end, where the GEMV's re-use of a weight row for the few rows of an
 //     expert runs out: 0.75 rows an expert for 4-bit (Qwen3-235B shapes 8
-//     tokens 129 / 149, 12 tokens 179 / 175, 20 tokens 273 / 226), 0.5 for
-//     6-bit (Qwen3-Next shapes 16 tokens 125 / 161, 24 tokens 233 / 169), 16
+//     tokens 129 / 148, 12 tokens 179 / 175, 20 tokens 273 / 226), a third for
+//     6-bit (Qwen3-Next shapes 8 tokens 69 / 88, 16 tokens 123 / 122, 24
+//     tokens 233 / 138), 16
 //     rows for reductions above 4096 (DeepSeek-V3 shapes 2 tokens 134 / 122,
 //     8 tokens 438 / 316); and 128 MiB of GEMV reads (rows x expert bytes), so
 //     that the extra launches pay (hidden 1024, 32 experts: 24 tokens 46 / 50,
@@ -219,7 +221,7 @@ bool stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int n_ids) 
     return false;
   if (rows > 32L * n_experts || rows * g->expert_bytes < (128L << 20)) return false;
   if (wide) return rows >= 16;
-  return g->bits == 4 ? 4 * rows >= 3L * n_experts : 2 * rows >= n_experts;
+  return g->bits == 4 ? 4 * rows >= 3L * n_experts : 3 * rows >= n_experts;
 }
 
 // Dispatch + the three projections (+ SwiGLU) for rows = n*kk flat rows.

@@ -18,16 +18,19 @@
 //     vector instructions a value, this 0.9): each group's product is scaled by
 //     its s in fp32, and (b - 128 s) * sum(x) is added by one fp32 MFMA per
 //     four groups, so no operand is rounded to bf16 but x itself.
-//   * The slices' fp32 partial sums meet in LDS once per 16 columns (double
-//     buffered, one LDS-only barrier, loads stay in flight across it).
-//   * Work is the flat list (tile, 16-column block), cut into equal
-//     contiguous ranges, one per resident block: every block streams the
-//     same number of bytes whatever the expert loads are.
+//   * The slices' fp32 partial sums meet in LDS once per step of four weight
+//     tiles (double buffered, one LDS-only barrier, loads stay in flight
+//     across it).  With one or two tiles a step, 16 columns stored at a time
+//     and 64-bit vector addresses, Qwen3-Next shapes took 169 us a layer at
+//     24 tokens and 415 at 1000, against 138 and 399.
+//   * Work is the flat list (row tile, step), cut into equal contiguous
+//     ranges, one per resident block: every block streams the same number of
+//     bytes whatever the expert loads are.
 //
 // Measured (Qwen3-235B shapes, 100 tokens, every expert active): gate/up 694
-// -> 187 us (4.8 TB/s of weights), down 395 -> 109 us (4.2 TB/s) against the
+// -> 186 us (4.9 TB/s of weights), down 395 -> 103 us (4.4 TB/s) against the
 // GEMV, which repeats its dot products for every row of an expert; the same
-// loads without arithmetic, reduction and stores take 157 and 82 us.  8 waves
+// loads without arithmetic, reduction and stores take 160 and 82 us.  8 waves
 // a CU at 256 registers: x takes 128 of them at 32 rows.
 #include <algorithm>
 #include <type_traits>
@@ -43,11 +46,13 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3_a4 __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kStreamRows = 32;   // rows of a dispatch tile
-constexpr int kCols = 16;         // weight rows (output columns) of a step
+constexpr int kCols = 16;         // weight rows (output columns) of a weight tile
+constexpr int kTiles = 4;         // weight tiles of a step (one reduction and barrier)
 constexpr int kPart = 256;        // floats of a 16 x 16 partial, in lane order
 
 struct StreamArgs {
@@ -62,7 +67,7 @@ struct StreamArgs {
   int out_cols;
   QProj p0, p1;
   void* out;              // gate/up: h (sorted rows); down: y (flat rows)
-  int out_vec;            // out is 16-byte aligned
+  int out_vec;            // bf16 out is 8-byte aligned
 };
 
 // One weight tile of a wave's slice: 16 rows x G groups.  The words stay in
@@ -104,21 +109,28 @@ struct WTile {
 // lower lanes holding the first group's two halves and the upper lanes the
 // second's; unpack_pair trades words between the wave's halves so that each
 // register then holds one group.  6-bit: 12 bytes a lane and group.
+// Addresses are a buffer resource over the expert's slot, a lane offset and a
+// scalar offset per tile (no vector arithmetic, no address registers).
 template <int BITS, int G>
-__device__ __forceinline__ void load_tile(WTile<BITS, G>& t, const uint8_t* w, uint32_t w_off,
-                                          const uint8_t* s, const uint8_t* b, uint32_t s_off) {
+__device__ __forceinline__ void load_tile(WTile<BITS, G>& t, __amdgpu_buffer_rsrc_t slot,
+                                          uint32_t w_off, uint32_t w, uint32_t s_off, uint32_t s,
+                                          uint32_t b) {
   using T = WTile<BITS, G>;
 #pragma unroll
-  for (int i = 0; i < T::kV; ++i)
-    t.w[i] = *reinterpret_cast<const typename T::V*>(w + w_off + (BITS == 4 ? 64 : 48) * i);
+  for (int i = 0; i < T::kV; ++i) {
+    if constexpr (BITS == 4)
+      t.w[i] = __builtin_amdgcn_raw_buffer_load_b128(slot, w_off + 64 * i, w, 0);
+    else
+      t.w[i] = __builtin_amdgcn_raw_buffer_load_b96(slot, w_off + 48 * i, w, 0);
+  }
 #pragma unroll
   for (int i = 0; i < T::kS4; ++i) {
-    t.s4[i] = *reinterpret_cast<const u32x4_a4*>(s + s_off + 16 * i);
-    t.b4[i] = *reinterpret_cast<const u32x4_a4*>(b + s_off + 16 * i);
+    t.s4[i] = __builtin_amdgcn_raw_buffer_load_b128(slot, s_off + 16 * i, s, 0);
+    t.b4[i] = __builtin_amdgcn_raw_buffer_load_b128(slot, s_off + 16 * i, b, 0);
   }
   if constexpr (T::kS3) {
-    t.s3 = *reinterpret_cast<const u32x3_a4*>(s + s_off + 16 * T::kS4);
-    t.b3 = *reinterpret_cast<const u32x3_a4*>(b + s_off + 16 * T::kS4);
+    t.s3 = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, s, 0);
+    t.b3 = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, b, 0);
   }
 }
 
@@ -254,38 +266,35 @@ __device__ __forceinline__ void tile_mfma(WTile<BITS, G>& t, const XTile<G> (&x)
 
 // A block's current tile.
 struct Seg {
-  const uint8_t* base;  // the expert's slot
-  int p0, m;            // first sorted row, rows
+  __amdgpu_buffer_rsrc_t slot;  // the expert's weights
+  int p0, m;                    // first sorted row, rows
 };
 
 template <int BITS, int G, int NSL, bool DUAL, bool F32>
 struct StreamKernel {
-  static constexpr int NP = DUAL ? 2 : 1;
   static constexpr int kThreads = 64 * NSL;
   static constexpr int kMaxMT = G <= 8 ? 2 : 1;  // 32 rows of x fit next to the ring
-  static constexpr int kLds = 2 * NP * kMaxMT * NSL * kPart;
-  // Output tile: two groups of 64 columns, rows padded by 16 bytes.
+  static constexpr int kStepCols = kTiles * kCols / (DUAL ? 2 : 1);  // output columns a step
+  // Partials of one weight tile: [row tile][slice][16 x 16]; the pad puts the
+  // tiles that 16 neighbouring threads of the reduction read on other banks.
+  static constexpr int kTilePart = kMaxMT * NSL * kPart + 16;
+  static constexpr int kLds = 2 * kTiles * kTilePart;
   using Out = std::conditional_t<F32, float, uint16_t>;
-  static constexpr int kOutRows = 16 * kMaxMT;
-  static constexpr int kOutPitch = 64 + 16 / int(sizeof(Out));
 
   // Weight tiles in flight: what fits in 256 registers next to x.
   template <int MT>
   static constexpr int ring() {
-    constexpr int per = WTile<BITS, G>::kRegs + G;
-    constexpr int room = 256 - (BITS == 4 ? 48 : MT == 1 ? 52 : 64) - MT * (8 * G + (G + 3) / 4) - NP * MT * 4;
-    constexpr int r = room / per;
-    constexpr int c = r > 4 ? 4 : r;
-    return c < NP ? NP : c / NP * NP;
+    constexpr int room = 256 - (BITS == 4 ? 56 : 72) - MT * (8 * G + (G + 3) / 4 + 4);
+    return 4 * (WTile<BITS, G>::kRegs + G) <= room ? 4 : 2;
   }
 
-  // Columns [ct0, ct1) (units of 16) of rows [r0, r0 + 16 MT) of the segment.
+  // Steps [st0, st1) of rows [r0, r0 + 16 MT) of the segment.  Tile t of a
+  // step: gate (even t) or up rows of 16 columns, or 16 down rows.
   template <int MT>
-  static __device__ __forceinline__ void run(const StreamArgs& a, const Seg& sg, int r0, int ct0,
-                                             int ct1, float* part, int& buf, Out* ot,
+  static __device__ __forceinline__ void run(const StreamArgs& a, const Seg& sg, int r0, int st0,
+                                             int st1, float* part, int& buf,
                                              const int32_t* s_row) {
     constexpr int E = ring<MT>();
-    constexpr int SR = E / NP;  // steps in flight
     const int lane = threadIdx.x & 63;
     const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 15, kq = lane >> 4;
@@ -294,22 +303,15 @@ struct StreamKernel {
     const uint32_t groups = uint32_t(a.cols) / 64;
     const uint32_t w_off = row * row_bytes + kq * (BITS == 4 ? 16 : 12);
     const uint32_t s_off = row * groups * 2;
-    const uint8_t* wb[2];
-    const uint8_t* sb[2];
-    const uint8_t* bb[2];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const QProj& q = p ? a.p1 : a.p0;
-      wb[p] = sg.base + q.w + slice * (G * 64 * BITS / 8);
-      sb[p] = sg.base + q.s + slice * (G * 2);
-      bb[p] = sg.base + q.b + slice * (G * 2);
-    }
     WTile<BITS, G> W[E];
-    auto load = [&](int e, int ct) {
-      const int p = e % NP;
-      load_tile<BITS, G>(W[e], wb[p] + size_t(ct) * kCols * row_bytes, w_off,
-                         sb[p] + size_t(ct) * kCols * groups * 2,
-                         bb[p] + size_t(ct) * kCols * groups * 2, s_off);
+    // tile t0 + e of a step into ring entry e (t0 even)
+    auto load = [&](int e, int t0, int step) {
+      const QProj& q = DUAL && (e & 1) ? a.p1 : a.p0;
+      const uint32_t r = (step * (kStepCols / kCols) + (DUAL ? (t0 + e) >> 1 : t0 + e)) * kCols;
+      const uint32_t g = slice * (G * 2) + r * groups * 2;
+      load_tile<BITS, G>(W[e], sg.slot, w_off,
+                         uint32_t(q.w) + slice * (G * 64 * BITS / 8) + r * row_bytes, s_off,
+                         uint32_t(q.s) + g, uint32_t(q.b) + g);
     };
     int ar[MT];
 #pragma unroll
@@ -318,7 +320,7 @@ struct StreamKernel {
       ar[mt] = DUAL ? a.order[r] / a.kk : r;
     }
 #pragma unroll
-    for (int e = 0; e < E; ++e) load(e, min(ct0 + e / NP, ct1 - 1));
+    for (int e = 0; e < E; ++e) load(e, 0, st0);
     __builtin_amdgcn_sched_barrier(0);
     XTile<G> x[MT];
 #pragma unroll
@@ -332,85 +334,68 @@ struct StreamKernel {
     // ring on every trip.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __builtin_amdgcn_sched_barrier(0);
-    for (int c = ct0; c < ct1; c += SR) {
+    for (int st = st0; st < st1; ++st) {
+      float* pb = part + buf * (kTiles * kTilePart);
+      const int next = min(st + 1, st1 - 1);  // past the range: the last step's again, unused
+      // One trip per ring length: each tile of a trip keeps its registers.
+#pragma unroll 1
+      for (int t0 = 0; t0 < kTiles; t0 += E) {
+        const int tn = t0 + E < kTiles ? t0 + E : 0;
+        const int sn = t0 + E < kTiles ? st : next;
 #pragma unroll
-      for (int v = 0; v < SR; ++v) {
-        // past the range: the last column again, the same values to the
-        // same place (an exit here would cost register copies that wait for
-        // the ring)
-        const int ct = min(c + v, ct1 - 1);
-        float* pb = part + buf * (NP * kMaxMT * NSL * kPart);
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
+        for (int e = 0; e < E; ++e) {
           f32x4 acc[MT];
-          tile_mfma<BITS, G, MT>(W[v * NP + p], x, kq, acc);
+          tile_mfma<BITS, G, MT>(W[e], x, kq, acc);
           __builtin_amdgcn_sched_barrier(0);
-          load(v * NP + p, min(ct + SR, ct1 - 1));
+          load(e, tn, sn);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              pb[((p * kMaxMT + mt) * NSL + slice) * kPart + 64 * r + lane] = acc[mt][r];
+              pb[(t0 + e) * kTilePart + (mt * NSL + slice) * kPart + 64 * r + lane] = acc[mt][r];
         }
-        block_lds_sync();
-        // the step before this one completed a 64-column group: it goes out
-        if ((ct & 3) == 0 && ct != ct0) flush(a, sg, r0, m, (ct >> 2) - 1, ct0, ct1, ot, s_row);
-        // Sum the slices into the output tile.  Rows past the tile repeat its
-        // last row and are never stored; threads beyond the outputs repeat
-        // the first ones'.
-        constexpr int J = MT * 256 > kThreads ? MT * 256 / kThreads : 1;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-          const int e = (int(threadIdx.x) + j * kThreads) % (MT * 256);
-          const int mt = e >> 8;
-          float v[2];
-#pragma unroll
-          for (int p = 0; p < NP; ++p) {
-            const float* q = pb + (p * kMaxMT + mt) * NSL * kPart + (e & 255);
-            v[p] = q[0];
-#pragma unroll
-            for (int sl = 1; sl < NSL; ++sl) v[p] += q[sl * kPart];
-          }
-          const float o = DUAL ? silu_fast(v[0]) * v[1] : v[0];
-          Out* d = ot + (ct & 4) / 4 * (kOutRows * kOutPitch) +
-                   (16 * mt + 4 * ((e >> 4) & 3) + ((e >> 6) & 3)) * kOutPitch +
-                   (ct & 3) * kCols + (e & 15);
-          if constexpr (F32)
-            *d = o;
-          else
-            *d = f2bf(o);
-        }
-        buf ^= 1;
       }
-    }
-    block_lds_sync();
-    flush(a, sg, r0, m, (ct1 - 1) >> 2, ct0, ct1, ot, s_row);
-  }
-
-  // Rows [0, m) of the 64-column group gi of the output tile, its columns
-  // within [ct0, ct1), as 16-byte pieces of whole lines.  (Stored by the step,
-  // 16 columns at a time, the short stores took a tenth of the gate/up
-  // launch: loads and stores share one counter, so the loads behind a store
-  // wait for its acknowledgement.)
-  static __device__ __forceinline__ void flush(const StreamArgs& a, const Seg& sg, int r0, int m,
-                                               int gi, int ct0, int ct1, const Out* ot,
-                                               const int32_t* s_row) {
-    constexpr int kPieces = 64 * sizeof(Out) / 16;
-    constexpr int kVals = 16 / sizeof(Out);
-    const Out* src = ot + (gi & 1) * (kOutRows * kOutPitch);
-    for (int i = threadIdx.x; i < m * kPieces; i += kThreads) {
-      const int r = i / kPieces, pc = i % kPieces;
-      const int ct = 4 * gi + pc / (kPieces / 4);
-      if (ct < ct0 || ct >= ct1) continue;
-      const int orow = DUAL ? sg.p0 + r0 + r : s_row[r0 + r];
-      Out* dst = static_cast<Out*>(a.out) + size_t(orow) * a.out_cols + 64 * gi + kVals * pc;
-      const Out* q = src + r * kOutPitch + kVals * pc;
-      if (a.out_vec)
-        *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(q);
-      else
+      block_lds_sync();
+      // Sum the slices: 4 columns of a row a thread, neighbouring threads
+      // along the row.
+      constexpr int kQuads = kStepCols / 4;
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));  // opaque: addresses recomputed here, not held across the loop
+      for (int i = tid; i < MT * 16 * kQuads; i += kThreads) {
+        const int c4 = i % kQuads, j = i / kQuads;
+        const int mt = j >> 4;
+        const int rr = 16 * mt + 4 * (j & 3) + ((j >> 2) & 3);
+        if (rr >= m) continue;
+        const float* q = pb + (DUAL ? 2 : 1) * (c4 >> 2) * kTilePart + mt * NSL * kPart +
+                         64 * ((j >> 2) & 3) + 16 * (j & 3) + 4 * (c4 & 3);
+        f32x4 v = *reinterpret_cast<const f32x4*>(q);
 #pragma unroll
-        for (int j = 0; j < kVals; ++j) dst[j] = q[j];
+        for (int sl = 1; sl < NSL; ++sl) v += *reinterpret_cast<const f32x4*>(q + sl * kPart);
+        if constexpr (DUAL) {
+          f32x4 u = *reinterpret_cast<const f32x4*>(q + kTilePart);
+#pragma unroll
+          for (int sl = 1; sl < NSL; ++sl)
+            u += *reinterpret_cast<const f32x4*>(q + kTilePart + sl * kPart);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = silu_fast(v[c]) * u[c];
+        }
+        const int orow = DUAL ? sg.p0 + r0 + rr : s_row[r0 + rr];
+        Out* dst = static_cast<Out*>(a.out) + size_t(orow) * a.out_cols + st * kStepCols + 4 * c4;
+        if constexpr (F32) {
+          *reinterpret_cast<f32x4*>(dst) = v;
+        } else {
+          const u32x2 o = {uint32_t(f2bf(v[0])) | uint32_t(f2bf(v[1])) << 16,
+                           uint32_t(f2bf(v[2])) | uint32_t(f2bf(v[3])) << 16};
+          if (DUAL || a.out_vec) {
+            *reinterpret_cast<u32x2*>(dst) = o;
+          } else {
+            dst[0] = Out(o[0]), dst[1] = Out(o[0] >> 16);
+            dst[2] = Out(o[1]), dst[3] = Out(o[1] >> 16);
+          }
+        }
+      }
+      buf ^= 1;
     }
   }
 };
@@ -419,35 +404,33 @@ template <int BITS, int G, int NSL, bool DUAL, bool F32>
 __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a) {
   using K = StreamKernel<BITS, G, NSL, DUAL, F32>;
   typedef const __attribute__((address_space(4))) int32_t ConstI32;
-  __shared__ float part[K::kLds];
-  __shared__ __attribute__((aligned(16))) typename K::Out ot[2 * K::kOutRows * K::kOutPitch];
+  __shared__ __attribute__((aligned(16))) float part[K::kLds];
   __shared__ int32_t s_row[2][kStreamRows];
-  const int n_ct = a.out_cols / kCols;
-  const int64_t total = int64_t(*(ConstI32*)a.n_tiles) * n_ct;
+  const int n_st = a.out_cols / K::kStepCols;
+  const int64_t total = int64_t(*(ConstI32*)a.n_tiles) * n_st;
   const int64_t u1 = total * (blockIdx.x + 1) / gridDim.x;
   int64_t u = total * blockIdx.x / gridDim.x;
   int buf = 0, par = 0;
   while (u < u1) {
-    const int tile = int(u / n_ct);
-    const int ct0 = int(u - int64_t(tile) * n_ct);
-    const int ct1 = int(min(int64_t(n_ct), ct0 + (u1 - u)));
-    u += ct1 - ct0;
+    const int tile = int(u / n_st);
+    const int st0 = int(u - int64_t(tile) * n_st);
+    const int st1 = int(min(int64_t(n_st), st0 + (u1 - u)));
+    u += st1 - st0;
     ConstI32* tl = (ConstI32*)(a.tiles + tile);
     const int slot = tl[0], first = tl[1], cnt = tl[2], off = tl[3];
     Seg sg;
     sg.p0 = off + first;
     sg.m = min(kStreamRows, cnt - first);
-    sg.base = a.slab + size_t(max(slot, 0)) * size_t(a.expert_bytes);
+    sg.slot = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(a.slab) + size_t(max(slot, 0)) * size_t(a.expert_bytes), 0,
+        uint32_t(a.expert_bytes), 0x00027000);
     if (slot < 0) {  // not resident: exact zero rows of y (streaming.py:715-719)
       if constexpr (!DUAL) {
-        const int nc = (ct1 - ct0) * kCols;
+        const int nc = (st1 - st0) * K::kStepCols;
         for (int i = threadIdx.x; i < sg.m * nc; i += K::kThreads) {
           const int r = i / nc;
-          const size_t o = size_t(a.order[sg.p0 + r]) * a.out_cols + ct0 * kCols + (i - r * nc);
-          if constexpr (F32)
-            static_cast<float*>(a.out)[o] = 0.0f;
-          else
-            static_cast<uint16_t*>(a.out)[o] = 0;
+          static_cast<typename K::Out*>(
+              a.out)[size_t(a.order[sg.p0 + r]) * a.out_cols + st0 * K::kStepCols + (i - r * nc)] = 0;
         }
       }
       continue;
@@ -459,12 +442,12 @@ __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a)
     }
     if constexpr (K::kMaxMT == 2) {
       if (sg.m > 16)
-        K::template run<2>(a, sg, 0, ct0, ct1, part, buf, ot, s_row[par]);
+        K::template run<2>(a, sg, 0, st0, st1, part, buf, s_row[par]);
       else
-        K::template run<1>(a, sg, 0, ct0, ct1, part, buf, ot, s_row[par]);
+        K::template run<1>(a, sg, 0, st0, st1, part, buf, s_row[par]);
     } else {
       for (int r0 = 0; r0 < sg.m; r0 += 16)
-        K::template run<1>(a, sg, r0, ct0, ct1, part, buf, ot, s_row[par]);
+        K::template run<1>(a, sg, r0, st0, st1, part, buf, s_row[par]);
     }
     par ^= 1;
   }
@@ -523,7 +506,8 @@ bool stream_covers(const pmoe_geom* g) {
 int stream_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                    const int32_t* order, const int4* tiles, const int32_t* n_tiles, uint16_t* h,
                    void* y, int y_f32, hipStream_t st) {
-  PMOE_REQUIRE(stream_covers(g), "stream: unsupported shape");
+  PMOE_REQUIRE(stream_covers(g) && g->expert_bytes < (int64_t(1) << 31),
+               "stream: unsupported shape");
   StreamArgs a{};
   a.slab = slab;
   a.expert_bytes = g->expert_bytes;
@@ -550,7 +534,7 @@ int stream_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, i
   a.out_cols = g->hidden;
   a.p0 = a.p1 = {g->off[PMOE_DOWN_W], g->off[PMOE_DOWN_S], g->off[PMOE_DOWN_B]};
   a.out = y;
-  a.out_vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  a.out_vec = (reinterpret_cast<uintptr_t>(y) & 7) == 0;
   ProfScope prof_scope(K_PREFILL_DOWN, st);
   if (y_f32)
     return g->bits == 4 ? launch_stream<4, false, true>(a, st)

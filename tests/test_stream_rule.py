@@ -10,7 +10,7 @@ import pytest
 
 @pytest.mark.parametrize("hidden,inter,bits,e,kk,form", [
     (4096, 1536, 4, 128, 8, {11: 0, 12: 1, 255: 1, 512: 1, 513: 0}),
-    (2048, 512, 6, 512, 11, {23: 0, 24: 1, 1489: 1, 1490: 0}),
+    (2048, 512, 6, 512, 11, {15: 0, 16: 1, 1489: 1, 1490: 0}),
     (7168, 2048, 4, 384, 9, {1: 0, 2: 1, 684: 1, 685: 0}),
     (1024, 512, 4, 32, 4, {37: 0, 38: 1, 255: 1, 256: 0}),
     (1024, 768, 4, 32, 4, {64: 0}),
