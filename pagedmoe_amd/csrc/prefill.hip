@@ -9,7 +9,8 @@
 //     tile's rows p (sorted positions) and 128 columns c of moe_intermediate;
 //   down_mfma_kernel:   y[order[p], d] = h_p . Wd[d] for 256 columns d of hidden.
 //
-// Work split (512 threads = 8 waves, two per SIMD): the tile's activation
+// Work split of the narrow form (512 threads = 8 waves, two per SIMD; the wide
+// form of large 4-bit layers is described at its code): the tile's activation
 // rows are staged through LDS one 64-wide quantization group at a time
 // (double buffered) and shared by the 8 waves; each wave owns 32 weight rows
 // (32 gate rows, 32 up rows, or 32 down rows: lane m of either lane half
@@ -908,6 +909,370 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
   }
 }
 
+// ---------------------------------------------------------------- wide form
+//
+// 4-bit, 128-row tiles, 64 weight rows a wave (two sets of 32), so each
+// activation fragment read from LDS feeds two MFMAs instead of one: at 32
+// rows a wave the fragment reads of a full tile take the whole LDS bandwidth
+// (8 waves x 16 KB a group against 128 bytes a cycle) beside the matrix cores'
+// 1024 cycles a group.  That leaves no registers for loads in flight (128
+// accumulators), so everything arrives by direct loads into LDS:
+//   A: the tile's rows, one group a stage, three buffers;
+//   W: each wave's own rows' packed words, two groups a unit, two buffers;
+//   S: each wave's own scales and biases, 8 groups a block, two buffers.
+// The loads are issued from inline assembly (they have no register results),
+// so the compiler, which has no vector memory operation of its own in the
+// loop, inserts no waits: one s_waitcnt per stage covers all three.  Past the
+// end the last stage, unit or block is loaded again, so the counts hold.
+//
+// Qwen3-235B shapes, rocprof, narrow -> wide: 16384 tokens gate/up 3781 ->
+// 3165 us, down 2110 -> 1785; 2048 tokens 670 -> 570 and 365 -> 317.  What is
+// left adds up rather than overlaps (the clock falls under this load): 16384
+// tokens' gate/up takes 2518 us without the dequantization, 2810 with the
+// fragments read once, 1717 without the MFMAs.  Measured and dropped: the
+// operand from (128 + q) pairs by dot products with (s, 0) and (0, s), 19
+// instead of 23 instructions per 8 values and the same bits (8192 tokens
+// 2851 -> 3190 us a layer); no fixed order of MFMAs and dequantization
+// (gate/up 3746 us); a higher wave priority for one wave of each SIMD (no
+// change).
+//
+// LDS rows are unpadded (a direct load writes 64 x 16 contiguous bytes), so
+// the 16-byte chunks of a row are permuted at the source instead: chunk c of A
+// row r sits at c ^ (r / 2 % 8), chunk c of W row r at c ^ (r / 4 % 4), and 16
+// consecutive rows' chunks fall on distinct banks.
+//
+// MFMAs per accumulator, their order and the dequantization are those of
+// gemm_tile, so the outputs are bit-identical.
+constexpr int kWideA = kTileM * 128;       // bytes of one A stage
+constexpr int kWideW = 64 * 64;            // bytes of one wave's W unit
+constexpr int kWideS = 2 * 64 * 16;        // bytes of one wave's S block
+constexpr int kWideOffW = 3 * kWideA;
+constexpr int kWideOffS = kWideOffW + (kThreads / 64) * 2 * kWideW;
+constexpr int kWideLds = kWideOffS + (kThreads / 64) * 2 * kWideS;
+constexpr int kWideGuCols = 256;           // moe_intermediate columns per gate/up block
+constexpr int kWideDnCols = 512;           // hidden columns per down block
+
+// 16 bytes a lane from base + voff to LDS bytes [lds, lds + 1024), lane l at
+// 16 l.  base and lds are wave-uniform.
+__device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t voff, const uint8_t* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(voff), "s"(base)
+               : "memory");
+}
+
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
+  return reinterpret_cast<const uint8_t*>(uint64_t(lo) | uint64_t(hi) << 32);
+}
+
+// The wave's weights: sets 0 and 1 of 32 rows, each row_bytes apart from
+// w[c]; scale and bias rows groups * 2 bytes apart from s[c], b[c].
+struct WideRows {
+  const uint8_t* w[2];
+  const uint8_t* s[2];
+  const uint8_t* b[2];
+};
+
+template <int NMB>
+__device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
+                                               const int32_t* order, int kk, int cols, int p0,
+                                               int m, const WideRows& wr, uint8_t* lds,
+                                               f32x16 (&acc)[2][kMB]) {
+  constexpr int kAIns = NMB > 2 ? 2 : 1;  // A loads a wave and stage, 8 rows each
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int last = n_groups - 1;
+  const int last_unit = (n_groups >> 1) - 1, last_blk = (n_groups >> 3) - 1;
+  const uint32_t row_bytes = uint32_t(cols) / 2;
+  typedef __attribute__((address_space(3))) uint8_t Lds8;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>((Lds8*)lds)));
+
+  // lane offsets of the loads
+  uint32_t a_off[kAIns];
+#pragma unroll
+  for (int i = 0; i < kAIns; ++i) {
+    const int r = 8 * (kAIns * wave + i) + (lane >> 3);  // LDS row
+    const int src = p0 + min(r, m - 1);                  // past the tile: its last row
+    a_off[i] = uint32_t(order ? order[src] / kk : src) * uint32_t(cols) * 2 +
+               16 * ((lane & 7) ^ ((r >> 1) & 7));
+  }
+  const uint32_t w_off = (lane >> 2) * row_bytes + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+  // rows 0-31 of set 0 in the lower lanes, of set 1 in the upper
+  const uint32_t sb_row = (lane & 31) * uint32_t(n_groups) * 2;
+  const uint32_t s_off = sb_row + (lane >> 5) * uint32_t(wr.s[1] - wr.s[0]);
+  const uint32_t b_off = sb_row + (lane >> 5) * uint32_t(wr.b[1] - wr.b[0]);
+  const uint32_t w_lds = lds0 + kWideOffW + wave * 2 * kWideW;
+  const uint32_t s_lds = lds0 + kWideOffS + wave * 2 * kWideS;
+
+  auto load_a = [&](int j, int buf) {
+    const uint8_t* base = act + size_t(min(j, last)) * 128;
+#pragma unroll
+    for (int i = 0; i < kAIns; ++i)
+      load_to_lds(lds0 + buf * kWideA + (kAIns * wave + i) * 1024, a_off[i], base);
+  };
+  auto load_w = [&](int u) {
+    const size_t at = size_t(min(u, last_unit)) * 64;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      load_to_lds(w_lds + (u & 1) * kWideW + i * 1024, w_off,
+                  wr.w[i >> 1] + at + size_t(i & 1) * 16 * row_bytes);
+  };
+  auto load_s = [&](int blk) {
+    const size_t at = size_t(min(blk, last_blk)) * 16;
+    load_to_lds(s_lds + (blk & 1) * kWideS, s_off, wr.s[0] + at);
+    load_to_lds(s_lds + (blk & 1) * kWideS + 1024, b_off, wr.b[0] + at);
+  };
+
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb) acc[c][mb] = f32x16{};
+  load_s(0);
+  load_w(0);
+  load_a(0, 0);
+  load_a(1, 1);
+  load_w(1);
+  load_s(1);
+  load_a(2, 2);
+
+  const int mrow = lane & 31, h = lane >> 5;
+  // lane addresses of the reads: A chunk 4 h + st of row mrow, W chunk h (+ 2
+  // for the unit's second group) of row mrow, S entry of the row
+  const uint8_t* a_rd = lds + mrow * 128;
+  const int a_swz = (mrow >> 1) & 7;
+  const uint8_t* w_rd = lds + kWideOffW + wave * 2 * kWideW + mrow * 64;
+  const int w_swz = (mrow >> 2) & 3;
+  const uint8_t* s_rd = lds + kWideOffS + wave * 2 * kWideS + mrow * 16;
+  SBlk S[2];
+  LaneWords<4> W[2];
+  bf16x8 A[2][NMB];
+  u32x4 B[2][4];
+  auto read_s = [&](int c, int blk) {
+    const uint8_t* q = s_rd + (blk & 1) * kWideS + c * 512;
+    S[c].s = *reinterpret_cast<const u32x4*>(q);
+    S[c].b = *reinterpret_cast<const u32x4*>(q + 1024);
+  };
+  // words of set c of a group: unit parity up, group gi of the unit
+  auto read_w = [&](int c, int up, int gi) {
+    const u32x4 t = *reinterpret_cast<const u32x4*>(w_rd + up * kWideW + c * 2048 +
+                                                    16 * ((2 * gi + h) ^ w_swz));
+    W[c].w[0] = t[0], W[c].w[1] = t[1], W[c].w[2] = t[2], W[c].w[3] = t[3];
+  };
+  auto read_a = [&](int mb, int st, int buf) {
+    A[st & 1][mb] = *reinterpret_cast<const bf16x8*>(a_rd + buf * kWideA + mb * 4096 +
+                                                     16 * ((4 * h + st) ^ a_swz));
+  };
+  // A(j + 1) has the next A stage and one W unit behind it in every stage, and
+  // the W unit and S block needed next are older: when no more than that is in
+  // flight they have landed, for this wave and, after the barrier, for all.
+  // (lgkmcnt: this wave's reads of the buffer that is given up have returned.)
+  auto arrive = [&]() {
+    if constexpr (kAIns == 2)
+      asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  arrive();
+#pragma unroll
+  for (int c = 0; c < 2; ++c) read_s(c, 0), read_w(c, 0, 0);
+#pragma unroll
+  for (int mb = 0; mb < NMB; ++mb) read_a(mb, 0, 0);
+  dequant_job<4>(W[0], S[0], 0, 0, B[0]);
+  dequant_job<4>(W[0], S[0], 0, 1, B[0]);
+  int buf = 0;  // of stage j
+  for (int j0 = 0; j0 < n_groups; j0 += 8) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int j = j0 + u;
+      const int nbuf = buf == 2 ? 0 : buf + 1;
+      const int un = (u + 1) & 7;  // the next group's scale entry
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        if (st == 1 && (u & 1)) {
+          // both groups of the unit are in registers (their last words were
+          // waited for in step 0): its buffer takes the unit after next, and
+          // after the first unit of a block, S's the block after next
+          load_w((j >> 1) + 2);
+          if (u == 1) load_s((j0 >> 3) + 2);
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+          for (int mb = 0; mb < NMB; ++mb) {
+            acc[c][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                A[st & 1][mb], __builtin_bit_cast(bf16x8, B[c][st]), acc[c][mb], 0, 0, 0);
+            if (c == 0 && st < 3) read_a(mb, st + 1, buf);
+            if (c == 0 && st == 3) {
+              if (mb == 0) {
+                // The last step's operands are in registers, so the next
+                // stage opens here, under this step's MFMAs: its first
+                // activations, words and operand are ready when it starts,
+                // and this stage's buffer takes the stage after the next two.
+                arrive();
+                load_a(j + 3, buf);
+                read_w(0, ((u + 1) >> 1) & 1, (u + 1) & 1);
+                if (u == 7) read_s(0, (j0 >> 3) + 1);
+              }
+              read_a(mb, 0, nbuf);
+            }
+            if (c == 1 && st == 3 && mb == 0) {
+              read_w(1, ((u + 1) >> 1) & 1, (u + 1) & 1);
+              if (u == 7) read_s(1, (j0 >> 3) + 1);
+            }
+            // the operand of the next set or step (or stage), 4 values after
+            // each of the set's first two MFMAs (both after one MFMA)
+#pragma unroll
+            for (int q = mb; q < (NMB == 1 ? 2 : mb < 2 ? mb + 1 : mb); ++q) {
+              if (c == 0)
+                dequant_job<4>(W[1], S[1], u, 2 * st + q, B[1]);
+              else if (st < 3)
+                dequant_job<4>(W[0], S[0], u, 2 * st + 2 + q, B[0]);
+              else
+                dequant_job<4>(W[0], S[0], un, q, B[0]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+      buf = nbuf;
+    }
+  }
+  // nothing may land in LDS after the caller starts to reuse it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+__device__ __forceinline__ void gemm_wide_any(int nmb, int n_groups, const uint8_t* act,
+                                              const int32_t* order, int kk, int cols, int p0,
+                                              int m, const WideRows& wr, uint8_t* lds,
+                                              f32x16 (&acc)[2][kMB]) {
+  switch (nmb) {
+    case 1: gemm_tile_wide<1>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    case 2: gemm_tile_wide<2>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    case 3: gemm_tile_wide<3>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    default: gemm_tile_wide<4>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+  }
+}
+
+// Wave w: gate rows (set 0) and up rows (set 1) of the same 32 columns, so
+// the SwiGLU needs no exchange.
+__global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const PrefillArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kWideLds];
+  TileInfo ti;
+  int cb;
+  if (!xcd_work<kTileM>(a, a.out_cols / kWideGuCols, ti, cb)) return;
+  if (ti.slot < 0) return;  // the down kernel writes this tile's zero rows
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const uint8_t* base = a.slab + size_t(ti.slot) * size_t(a.expert_bytes);
+  const size_t row_bytes = size_t(a.cols) / 2;
+  const int groups = a.cols / 64;
+  const int col0 = cb * kWideGuCols + wave * 32;
+  WideRows wr;
+  wr.w[0] = uniform_ptr(base + a.w0 + col0 * row_bytes);
+  wr.w[1] = uniform_ptr(base + a.w1 + col0 * row_bytes);
+  wr.s[0] = uniform_ptr(base + a.s0 + size_t(col0) * groups * 2);
+  wr.s[1] = uniform_ptr(base + a.s1 + size_t(col0) * groups * 2);
+  wr.b[0] = uniform_ptr(base + a.b0 + size_t(col0) * groups * 2);
+  wr.b[1] = uniform_ptr(base + a.b1 + size_t(col0) * groups * 2);
+  f32x16 acc[2][kMB];
+  const int nmb = __builtin_amdgcn_readfirstlane((ti.m + 31) >> 5);
+  gemm_wide_any(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), a.order, a.kk, a.cols, ti.p0,
+                ti.m, wr, lds, acc);
+  const int h = lane >> 5;
+  uint16_t* hout = static_cast<uint16_t*>(a.out) + col0 + (lane & 31);
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = mb * 32 + acc_row(r, h);
+      if (row < ti.m)
+        hout[size_t(ti.p0 + row) * a.out_cols] = f2bf(silu_fast(acc[0][mb][r]) * acc[1][mb][r]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kWideLds];
+  __shared__ int32_t s_ord[kTileM];
+  TileInfo ti;
+  int cb;
+  if (!xcd_work<kTileM>(a, a.out_cols / kWideDnCols, ti, cb)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (ti.slot < 0) {  // not resident: exact zero rows (streaming.py:715-719)
+    for (int row = 0; row < ti.m; ++row) {
+      const size_t o = size_t(a.order[ti.p0 + row]) * a.out_cols + cb * kWideDnCols + threadIdx.x;
+      if (a.out_f32)
+        static_cast<float*>(a.out)[o] = 0.0f;
+      else
+        static_cast<uint16_t*>(a.out)[o] = 0;
+    }
+    return;
+  }
+  const uint8_t* base = a.slab + size_t(ti.slot) * size_t(a.expert_bytes);
+  const size_t row_bytes = size_t(a.cols) / 2;
+  const int groups = a.cols / 64;
+  const int col0 = cb * kWideDnCols + wave * 64;
+  WideRows wr;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    wr.w[c] = uniform_ptr(base + a.w0 + (col0 + 32 * c) * row_bytes);
+    wr.s[c] = uniform_ptr(base + a.s0 + size_t(col0 + 32 * c) * groups * 2);
+    wr.b[c] = uniform_ptr(base + a.b0 + size_t(col0 + 32 * c) * groups * 2);
+  }
+  if (int(threadIdx.x) < ti.m) s_ord[threadIdx.x] = a.order[ti.p0 + threadIdx.x];
+  f32x16 acc[2][kMB];
+  const int nmb = __builtin_amdgcn_readfirstlane((ti.m + 31) >> 5);
+  gemm_wide_any(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), nullptr, 1, a.cols, ti.p0,
+                ti.m, wr, lds, acc);
+  const int h = lane >> 5;
+  if (a.out_f32 || !a.out_vec) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = mb * 32 + acc_row(r, h);
+          if (row < ti.m) {
+            const size_t o = size_t(s_ord[row]) * a.out_cols + col0 + 32 * c + (lane & 31);
+            if (a.out_f32)
+              static_cast<float*>(a.out)[o] = acc[c][mb][r];
+            else
+              static_cast<uint16_t*>(a.out)[o] = f2bf(acc[c][mb][r]);
+          }
+        }
+    return;
+  }
+  // bf16 rows go out through LDS as 16-byte pieces, as in down_mfma_kernel
+  constexpr int kEp = kWideDnCols + 8;
+  constexpr int kPieces = kWideDnCols / 8;
+  static_assert(kTileM * kEp * 2 <= kWideLds, "output tile in LDS");
+  uint16_t* ot = reinterpret_cast<uint16_t*>(lds);
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+      if (mb < nmb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          ot[(mb * 32 + acc_row(r, h)) * kEp + wave * 64 + 32 * c + (lane & 31)] =
+              f2bf(acc[c][mb][r]);
+  __syncthreads();
+  uint16_t* out = static_cast<uint16_t*>(a.out) + cb * kWideDnCols;
+  for (int q = threadIdx.x; q < ti.m * kPieces; q += kThreads) {
+    const int row = q / kPieces, pc = q - row * kPieces;
+    *reinterpret_cast<uint4*>(out + size_t(s_ord[row]) * a.out_cols + 8 * pc) =
+        *reinterpret_cast<const uint4*>(ot + row * kEp + 8 * pc);
+  }
+}
+
 }  // namespace
 
 // 32-row tiles at two blocks per CU when the routed experts see at most 32
@@ -941,9 +1306,25 @@ bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids) {
   return rows >= 1024 && rows >= 16L * n_ids;
 }
 
+// The wide 128-row form (4-bit) once the narrow one's gate/up items, 128
+// columns each, are more than one a CU: below that a launch takes one block's
+// time, and the narrow block's is shorter.  Measured us a layer, narrow / wide:
+// hidden 1024, 32 experts 1400 tokens 67 / 78, 2000 tokens 98 / 81, 16000
+// tokens 411 / 366; Qwen3-235B shapes 520 tokens 491 / 492, 2048 tokens
+// 1044 / 967, 8192 tokens 3346 / 2851; DeepSeek-V3 shapes 2048 tokens
+// 3717 / 3372.  Tiles are estimated as full ones plus half of one an expert.
+// PMOE_PREFILL_WIDE=1 / 0 pins either (same outputs).
+bool prefill_wide(const pmoe_geom* g, int n, int kk, int n_experts) {
+  const char* v = getenv("PMOE_PREFILL_WIDE");
+  if (v && (v[0] == '0' || v[0] == '1')) return v[0] == '1';
+  const long tiles = long(n) * kk / kTileM + n_experts / 2;
+  return tiles * (g->inter / kGuCols) > 256;
+}
+
 int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                     const int32_t* order, const int4* tiles, const int32_t* n_tiles, int tile_m,
-                    int max_tiles, uint16_t* h, void* y, int y_f32, hipStream_t st) {
+                    int max_tiles, int n_experts, uint16_t* h, void* y, int y_f32,
+                    hipStream_t st) {
   PMOE_REQUIRE(tile_m == 32 || tile_m == kTileM, "prefill: tile height must be 32 or 128");
   PMOE_REQUIRE(g->inter % 512 == 0 && g->hidden % 512 == 0,
                "prefill: hidden and inter must be multiples of 512");
@@ -952,6 +1333,7 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
                    int64_t(n) * kk * g->inter < (int64_t(1) << 31),
                "prefill: activations exceed 2^31 elements");
   const bool small = tile_m == 32;
+  const bool wide = prefill_wide(g, n, kk, n_experts);
   PrefillArgs a{};
   a.slab = slab;
   a.expert_bytes = g->expert_bytes;
@@ -977,6 +1359,8 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
     ProfScope prof_scope(K_PREFILL_GATEUP, st);
     if (g->bits == 4 && small)
       gateup_mfma_kernel<4, 1><<<grid, kThreads, 0, st>>>(a);
+    else if (g->bits == 4 && wide)
+      gateup_wide_kernel<<<(g->inter / kWideGuCols * max_tiles + 7) / 8 * 8, kThreads, 0, st>>>(a);
     else if (g->bits == 4)
       gateup_mfma_kernel<4, kMB><<<grid, kThreads, 0, st>>>(a);
     else if (small)
@@ -1002,6 +1386,8 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
     ProfScope prof_scope(K_PREFILL_DOWN, st);
     if (g->bits == 4 && small)
       down_mfma_kernel<4, 1><<<grid, kThreads, 0, st>>>(a);
+    else if (g->bits == 4 && wide)
+      down_wide_kernel<<<(g->hidden / kWideDnCols * max_tiles + 7) / 8 * 8, kThreads, 0, st>>>(a);
     else if (g->bits == 4)
       down_mfma_kernel<4, kMB><<<grid, kThreads, 0, st>>>(a);
     else if (small)

@@ -1,0 +1,80 @@
+"""GPU: the wide 128-row prefill form (direct loads into LDS, two weight sets a
+wave) against the narrow one, bit for bit, and the float64 oracle: rows per
+expert around its 32-row blocks and 128-row tiles, reductions of one scale
+block (8 groups) and more, absent experts, dropped ids, and an output that is
+not 16-byte aligned."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import pmoe_oracle as O
+from tests.test_gpu_stream import _ids, _setup
+from tests.util import bits_to_bf16_tensor, check_close
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+COUNTS = [300, 129, 128, 127, 97, 96, 1, 31, 32, 33, 64, 65, 90]
+
+
+@pytest.mark.parametrize("hidden,inter", [(1024, 512), (2048, 1536), (512, 1024), (4096, 512)])
+def test_wide_matches_narrow_and_oracle(hidden, inter, monkeypatch):
+    from pagedmoe_amd import kernels as K
+    monkeypatch.setenv("PMOE_STREAM", "0")
+    monkeypatch.setenv("PMOE_PREFILL_SMALL", "0")
+    n, k, e = 330, 4, len(COUNTS)
+    g, slab, experts = _setup(hidden, inter, 4, e, 60)
+    rng = np.random.default_rng(hidden + inter)
+    xb = O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32))
+    ids = _ids(COUNTS, k, rng, n)
+    table = torch.arange(e, dtype=torch.int32, device=DEV)
+    table[12] = -1
+    x, inds = bits_to_bf16_tensor(xb, DEV), torch.from_numpy(ids).to(DEV)
+    got = []
+    for pin in ("0", "1"):
+        monkeypatch.setenv("PMOE_PREFILL_WIDE", pin)
+        got.append(K.switch_glu(g, slab.buf, table, e, x, inds))
+    assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
+    y = got[1].float().cpu().numpy()
+    gone = (ids < 0) | (ids == 12)
+    assert (y[gone] == 0).all()
+    ref = O.switch_glu_f64(xb, np.where(gone, 0, ids), experts)
+    check_close(y[~gone], ref[~gone], f"wide {hidden}x{inter}")
+    # unaligned output rows take the element-wise stores
+    big = torch.full((n * k * hidden + 8,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    un = big[1:1 + n * k * hidden]
+    from pagedmoe_amd._lib import check, lib
+    ws = K.moe_workspace(g, n, k, 0, e, x.device)
+    check(lib().pmoe_switch_glu(ctypes.byref(g), K._ptr(slab.buf), K._table_ptr(table), e,
+                                K._ptr(x), K._ptr(inds), n, k, ctypes.c_void_p(un.data_ptr()),
+                                K._ptr(ws), ws.numel(), K._stream()), "pmoe_switch_glu")
+    torch.cuda.synchronize()
+    assert torch.equal(got[1].reshape(-1).view(torch.int16), un.view(torch.int16))
+    assert torch.isnan(big[0]) and torch.isnan(big[-7:]).all()
+    slab.release()
+
+
+def test_wide_block_in_a_graph(monkeypatch):
+    """The whole block in the wide form, replayed from a HIP graph."""
+    from pagedmoe_amd import kernels as K
+    monkeypatch.setenv("PMOE_PREFILL_WIDE", "1")
+    g, slab, _ = _setup(1024, 512, 4, 8, 61)
+    rng = np.random.default_rng(62)
+    gw = bits_to_bf16_tensor(O.bf16_round(rng.standard_normal((8, 1024), dtype=np.float32)
+                                          * np.float32(0.02)), DEV)
+    x = bits_to_bf16_tensor(O.bf16_round(rng.standard_normal((520, 1024), dtype=np.float32)), DEV)
+    table = torch.arange(8, dtype=torch.int32, device=DEV)
+    rc = K.route_cfg("softmax", 8, 2)
+    eager = K.moe_block(g, rc, slab.buf, table, gw, x)[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, _, _ = K.moe_block(g, rc, slab.buf, table, gw, x)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
+    slab.release()
