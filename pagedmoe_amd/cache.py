@@ -20,6 +20,7 @@ import torch
 
 from . import config
 from ._lib import Geom, PmoeError, SlabStats, check, lib
+from .kernels import _stream
 from .slab import SlabStore
 
 
@@ -269,7 +270,7 @@ class ExpertCache:
 
     def sync_table(self, layer_key) -> bool:
         """Republish the layer's device row if it is stale; True if it was."""
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = self._stream()
         r = lib().pmoe_slab_sync_table(self._h, self.layer_index(layer_key), stream)
         if r < 0:
             check(r, "pmoe_slab_sync_table")
@@ -297,7 +298,7 @@ class ExpertCache:
         return self.routed_slots + self.layer_index(layer_key)
 
     def publish(self, layer_key) -> None:
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = self._stream()
         check(lib().pmoe_slab_publish(self._h, self.layer_index(layer_key), stream),
               "pmoe_slab_publish")
 
@@ -326,7 +327,7 @@ class ExpertCache:
             self.spec_log.append(("fetch", layer_key, list(ids)))
         arr = (ctypes.c_int32 * max(1, len(ids)))(*ids)
         nm = ctypes.c_int()
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = self._stream()
         check(lib().pmoe_slab_fetch(self._h, self._ce, ctypes.byref(self.geom),
                                     ctypes.c_void_p(self.slab.data_ptr),
                                     ctypes.c_void_p(self.host_store.address),
@@ -541,7 +542,7 @@ class ExpertCache:
 
     @staticmethod
     def _stream():
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _stream()
 
     def sync_copies(self) -> None:
         if self._ce.value:

@@ -31,7 +31,11 @@ def _ptr(t):
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current device's current stream.  Read as a raw handle: building
+    torch's Stream object takes 4 us, and a paged decode layer asks six times."""
+    if not torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _need(t, dtype, name, ndim=None):
@@ -219,9 +223,10 @@ def raise_workspace_errors() -> None:
     PmoeError if a grid barrier of the one-launch decode timed out (those
     layer outputs are NaN).  The failed workspace is re-initialised first,
     so the next call runs normally."""
-    words = {ws.data_ptr(): int(_ERR_HOST.get(ws.data_ptr(),
-                                              torch.zeros(1, dtype=torch.int32))[0])
-             for ws in _live_moe_workspaces()}
+    words = {}
+    for ws in _live_moe_workspaces():
+        host = _ERR_HOST.get(ws.data_ptr())
+        words[ws.data_ptr()] = 0 if host is None else host.item()
     bad = [ws for ws in _live_moe_workspaces() if words[ws.data_ptr()] != 0]
     if not bad:
         return

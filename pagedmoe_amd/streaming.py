@@ -67,6 +67,11 @@ class QuantizedSwitchGLU(nn.Module):
         return y.reshape(*lead, self.hidden)
 
 
+# Routed ids made distinct on the host rather than on the device (a call's
+# flat [N * K]): 25 us of host time at most, against two synchronisations.
+HOST_UNIQUE_IDS = 1024
+
+
 class StreamedSwitchGLU(nn.Module):
     """The seam: same call contract as QuantizedSwitchGLU, experts paged
     into the cache's slab on demand.
@@ -109,7 +114,12 @@ class StreamedSwitchGLU(nn.Module):
         sync also carries the MoE workspaces' error words: a timed-out grid
         barrier of an earlier one-launch decode raises here."""
         K.note_workspace_errors()
-        ids = [e for e in torch.unique(indices.reshape(-1)).tolist() if 0 <= e < self.n_experts]
+        flat = indices.reshape(-1)
+        # Up to HOST_UNIQUE_IDS ids cross as they are: torch.unique sorts them
+        # in seven launches and synchronises once more on their count.
+        found = (set(flat.tolist()) if flat.numel() <= HOST_UNIQUE_IDS
+                 else torch.unique(flat).tolist())
+        ids = sorted(e for e in found if 0 <= e < self.n_experts)
         K.raise_workspace_errors()
         if self.ring is not None:
             self.ring.collect_predictions()   # they rode this sync
