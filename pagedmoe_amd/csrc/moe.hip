@@ -124,6 +124,32 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   *reinterpret_cast<uint4*>(out + size_t(n) * d + d0) = o;
 }
 
+// Same reduction over fp32 per-slot outputs (the streamed block path), 4 outputs
+// per thread: combine_y_kernel's fma chain, the weights from the routing
+// launch and the shared expert's gate logits.
+__global__ __launch_bounds__(256) void combine_f32_kernel(const float* __restrict__ y,
+                                                          const float* __restrict__ w,
+                                                          const float* __restrict__ shared_logit,
+                                                          int k, int kk, int d,
+                                                          uint16_t* __restrict__ out) {
+  const int n = blockIdx.y;
+  const int d0 = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (d0 >= d) return;
+  float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c = 0; c < kk; ++c) {
+    const float wt =
+        c < k ? w[size_t(n) * k + c] : shared_logit ? psigmoid(shared_logit[n]) : 1.0f;
+    const float4 v = *reinterpret_cast<const float4*>(y + (size_t(n) * kk + c) * d + d0);
+    a[0] = __builtin_fmaf(wt, v.x, a[0]);
+    a[1] = __builtin_fmaf(wt, v.y, a[1]);
+    a[2] = __builtin_fmaf(wt, v.z, a[2]);
+    a[3] = __builtin_fmaf(wt, v.w, a[3]);
+  }
+  uint16_t* o = out + size_t(n) * d + d0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = f2bf(a[i]);
+}
+
 // Same reduction over bf16 per-slot outputs (the seam's [N, K, D]), for
 // callers that ran the experts in several passes.
 __global__ __launch_bounds__(256) void combine_bf16_kernel(const uint16_t* __restrict__ y,
@@ -373,14 +399,40 @@ int decode_block(const pmoe_geom* g, const pmoe_route_cfg* rc, const uint8_t* sl
                                 out, w.sync, st);
     if (r2 != kDecodeFusedDeclined) return r2;
   }
+  // streamed experts into fp32 per-slot rows (a pinned decode form compares
+  // the GEMV paths and keeps them)
   if (n > 1 && !getenv("PMOE_DECODE_FUSED") && stream_wanted(g, n, kk, e, e + shared)) {
-    // (a pinned decode form compares the GEMV paths) the router launch (routing in its last block), the dispatch of its
-    // picks, the streamed experts into fp32 per-slot rows, the combine
-    int r = decode_route(gu, rt, inds_out, w_out, w.record, ri, st);
-    if (r) return r;
+    // Up to 12 tokens the router launch's last block routes, one token a wave
+    // and round; beyond, its rounds cost more than a routing launch with a wave
+    // for every token (us a layer, last block / launch: Qwen3-235B shapes 12
+    // tokens 180 / 183, 16 tokens 199 / 197, 29 tokens 272 / 264; Qwen3-Next
+    // shapes 23 tokens 144 / 134).
+    constexpr int kRouteTailTokens = 12;
+    int r;
+    if (n <= kRouteTailTokens) {
+      r = decode_route(gu, rt, inds_out, w_out, w.record, ri, st);
+      if (r) return r;
+    } else {
+      r = router_logits(x, gate_w, logit_bias, n, g->hidden, e, w.logits, st);
+      if (r) return r;
+      r = rc->scoring == PMOE_SCORE_SOFTMAX
+              ? route_softmax(w.logits, n, e, k, rc->norm_topk_prob, inds_out, w_out, st)
+              : route_sigmoid(w.logits, score_bias, n, e, rc->n_group, rc->topk_group, k,
+                              rc->norm_topk_prob, rc->routed_scale, inds_out, w_out, st);
+      if (r) return r;
+      if (extra) {
+        r = router_logits(x, extra, nullptr, n, g->hidden, 1, w.shared_logit, st);
+        if (r) return r;
+      }
+    }
     r = run_experts(g, slab, table, e, shared_slot, x, inds_out, n, k, kk, n, w, w.y, 1, st);
     if (r) return r;
-    return decode_combine(w.y, w.record, n, kk, g->hidden, out, st);
+    if (n <= kRouteTailTokens) return decode_combine(w.y, w.record, n, kk, g->hidden, out, st);
+    ProfScope prof_scope(K_COMBINE, st);
+    combine_f32_kernel<<<dim3((g->hidden / 4 + 255) / 256, n), 256, 0, st>>>(
+        w.y, w_out, extra ? w.shared_logit : nullptr, k, kk, g->hidden, out);
+    PMOE_LAUNCH_CHECK("combine_f32_kernel");
+    return PMOE_OK;
   }
   dn.out = w.y;  // fp32 per-slot outputs when the down runs expert-split
   return decode_routed(gu, dn, rt, g->bits, inds_out, w_out, out, w.record, ri, st);

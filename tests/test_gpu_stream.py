@@ -97,7 +97,7 @@ def test_stream_unaligned_output_matches_aligned(monkeypatch):
     slab.release()
 
 
-@pytest.mark.parametrize("bits,n", [(4, 2), (4, 17), (6, 50)])
+@pytest.mark.parametrize("bits,n", [(4, 2), (4, 12), (4, 13), (4, 17), (6, 50)])
 def test_stream_block_vs_oracle(bits, n, monkeypatch):
     """The whole block with a gated shared expert (its rows are every token:
     at 50 tokens two tiles), eager and replayed from a HIP graph."""
