@@ -10,7 +10,7 @@
 //   down_mfma_kernel:   y[order[p], d] = h_p . Wd[d] for 256 columns d of hidden.
 //
 // Work split of the narrow form (512 threads = 8 waves, two per SIMD; the wide
-// form of large 4-bit layers is described at its code): the tile's activation
+// form of larger layers is described at its code): the tile's activation
 // rows are staged through LDS one 64-wide quantization group at a time
 // (double buffered) and shared by the 8 waves; each wave owns 32 weight rows
 // (32 gate rows, 32 up rows, or 32 down rows: lane m of either lane half
@@ -911,14 +911,15 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
 
 // ---------------------------------------------------------------- wide form
 //
-// 4-bit, 128-row tiles, 64 weight rows a wave (two sets of 32), so each
+// 128-row tiles, 64 weight rows a wave (two sets of 32), so each
 // activation fragment read from LDS feeds two MFMAs instead of one: at 32
 // rows a wave the fragment reads of a full tile take the whole LDS bandwidth
 // (8 waves x 16 KB a group against 128 bytes a cycle) beside the matrix cores'
 // 1024 cycles a group.  That leaves no registers for loads in flight (128
 // accumulators), so everything arrives by direct loads into LDS:
 //   A: the tile's rows, one group a stage, three buffers;
-//   W: each wave's own rows' packed words, two groups a unit, two buffers;
+//   W: each wave's own rows' packed words, two groups a unit and two buffers
+//     (4-bit), or one group (three 16-byte chunks a row) and three (6-bit);
 //   S: each wave's own scales and biases, 8 groups a block, two buffers.
 // The loads are issued from inline assembly (they have no register results),
 // so the compiler, which has no vector memory operation of its own in the
@@ -944,11 +945,16 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
 // MFMAs per accumulator, their order and the dequantization are those of
 // gemm_tile, so the outputs are bit-identical.
 constexpr int kWideA = kTileM * 128;       // bytes of one A stage
-constexpr int kWideW = 64 * 64;            // bytes of one wave's W unit
 constexpr int kWideS = 2 * 64 * 16;        // bytes of one wave's S block
 constexpr int kWideOffW = 3 * kWideA;
-constexpr int kWideOffS = kWideOffW + (kThreads / 64) * 2 * kWideW;
-constexpr int kWideLds = kWideOffS + (kThreads / 64) * 2 * kWideS;
+template <int BITS>
+struct Wide {
+  static constexpr int kW = BITS == 4 ? 64 * 64 : 64 * 48;  // bytes of one wave's W unit
+  static constexpr int kWBufs = BITS == 4 ? 2 : 3;
+  static constexpr int kWWave = kWBufs * kW;
+  static constexpr int kOffS = kWideOffW + (kThreads / 64) * kWWave;
+  static constexpr int kLds = kOffS + (kThreads / 64) * 2 * kWideS;
+};
 constexpr int kWideGuCols = 256;           // moe_intermediate columns per gate/up block
 constexpr int kWideDnCols = 512;           // hidden columns per down block
 
@@ -976,17 +982,18 @@ struct WideRows {
   const uint8_t* b[2];
 };
 
-template <int NMB>
+template <int BITS, int NMB>
 __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
                                                const int32_t* order, int kk, int cols, int p0,
                                                int m, const WideRows& wr, uint8_t* lds,
                                                f32x16 (&acc)[2][kMB]) {
   constexpr int kAIns = NMB > 2 ? 2 : 1;  // A loads a wave and stage, 8 rows each
+  using L = Wide<BITS>;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int last = n_groups - 1;
-  const int last_unit = (n_groups >> 1) - 1, last_blk = (n_groups >> 3) - 1;
-  const uint32_t row_bytes = uint32_t(cols) / 2;
+  const int last_unit = (BITS == 4 ? n_groups >> 1 : n_groups) - 1, last_blk = (n_groups >> 3) - 1;
+  const uint32_t row_bytes = uint32_t(cols) * BITS / 8;
   typedef __attribute__((address_space(3))) uint8_t Lds8;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>((Lds8*)lds)));
 
@@ -999,13 +1006,24 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
     a_off[i] = uint32_t(order ? order[src] / kk : src) * uint32_t(cols) * 2 +
                16 * ((lane & 7) ^ ((r >> 1) & 7));
   }
-  const uint32_t w_off = (lane >> 2) * row_bytes + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+  // 4-bit: row lane / 4 (+ 16 a load), permuted chunk; 6-bit: chunk q of the
+  // unit's 192 is row q / 3, chunk q % 3, rows 32-63 in set 1
+  uint32_t w_off[BITS == 4 ? 1 : 3];
+  if constexpr (BITS == 4) {
+    w_off[0] = (lane >> 2) * row_bytes + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t q = 64 * i + lane, r = q / 3;
+      w_off[i] = (r & 31) * row_bytes + (r >> 5) * uint32_t(wr.w[1] - wr.w[0]) + 16 * (q - 3 * r);
+    }
+  }
   // rows 0-31 of set 0 in the lower lanes, of set 1 in the upper
   const uint32_t sb_row = (lane & 31) * uint32_t(n_groups) * 2;
   const uint32_t s_off = sb_row + (lane >> 5) * uint32_t(wr.s[1] - wr.s[0]);
   const uint32_t b_off = sb_row + (lane >> 5) * uint32_t(wr.b[1] - wr.b[0]);
-  const uint32_t w_lds = lds0 + kWideOffW + wave * 2 * kWideW;
-  const uint32_t s_lds = lds0 + kWideOffS + wave * 2 * kWideS;
+  const uint32_t w_lds = lds0 + kWideOffW + wave * L::kWWave;
+  const uint32_t s_lds = lds0 + L::kOffS + wave * 2 * kWideS;
 
   auto load_a = [&](int j, int buf) {
     const uint8_t* base = act + size_t(min(j, last)) * 128;
@@ -1013,12 +1031,19 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
     for (int i = 0; i < kAIns; ++i)
       load_to_lds(lds0 + buf * kWideA + (kAIns * wave + i) * 1024, a_off[i], base);
   };
-  auto load_w = [&](int u) {
-    const size_t at = size_t(min(u, last_unit)) * 64;
+  auto load_w = [&](int u, int buf) {
+    if constexpr (BITS == 4) {
+      const size_t at = size_t(min(u, last_unit)) * 64;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      load_to_lds(w_lds + (u & 1) * kWideW + i * 1024, w_off,
-                  wr.w[i >> 1] + at + size_t(i & 1) * 16 * row_bytes);
+      for (int i = 0; i < 4; ++i)
+        load_to_lds(w_lds + buf * L::kW + i * 1024, w_off[0],
+                    wr.w[i >> 1] + at + size_t(i & 1) * 16 * row_bytes);
+    } else {
+      const size_t at = size_t(min(u, last_unit)) * 48;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        load_to_lds(w_lds + buf * L::kW + i * 1024, w_off[i], wr.w[0] + at);
+    }
   };
   auto load_s = [&](int blk) {
     const size_t at = size_t(min(blk, last_blk)) * 16;
@@ -1031,23 +1056,25 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
 #pragma unroll
     for (int mb = 0; mb < kMB; ++mb) acc[c][mb] = f32x16{};
   load_s(0);
-  load_w(0);
+  load_w(0, 0);
   load_a(0, 0);
   load_a(1, 1);
-  load_w(1);
+  load_w(1, 1);
   load_s(1);
   load_a(2, 2);
+  if constexpr (BITS == 6) load_w(2, 2);
 
   const int mrow = lane & 31, h = lane >> 5;
   // lane addresses of the reads: A chunk 4 h + st of row mrow, W chunk h (+ 2
   // for the unit's second group) of row mrow, S entry of the row
   const uint8_t* a_rd = lds + mrow * 128;
   const int a_swz = (mrow >> 1) & 7;
-  const uint8_t* w_rd = lds + kWideOffW + wave * 2 * kWideW + mrow * 64;
+  const uint8_t* w_rd = lds + kWideOffW + wave * L::kWWave +
+                        (BITS == 4 ? mrow * 64 : mrow * 48 + 24 * h);
   const int w_swz = (mrow >> 2) & 3;
-  const uint8_t* s_rd = lds + kWideOffS + wave * 2 * kWideS + mrow * 16;
+  const uint8_t* s_rd = lds + L::kOffS + wave * 2 * kWideS + mrow * 16;
   SBlk S[2];
-  LaneWords<4> W[2];
+  LaneWords<BITS> W[2];
   bf16x8 A[2][NMB];
   u32x4 B[2][4];
   auto read_s = [&](int c, int blk) {
@@ -1055,25 +1082,29 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
     S[c].s = *reinterpret_cast<const u32x4*>(q);
     S[c].b = *reinterpret_cast<const u32x4*>(q + 1024);
   };
-  // words of set c of a group: unit parity up, group gi of the unit
-  auto read_w = [&](int c, int up, int gi) {
-    const u32x4 t = *reinterpret_cast<const u32x4*>(w_rd + up * kWideW + c * 2048 +
-                                                    16 * ((2 * gi + h) ^ w_swz));
-    W[c].w[0] = t[0], W[c].w[1] = t[1], W[c].w[2] = t[2], W[c].w[3] = t[3];
+  // words of set c of a group: buffer wb, group gi of a 4-bit unit
+  auto read_w = [&](int c, int wb, int gi) {
+    if constexpr (BITS == 4) {
+      const u32x4 t = *reinterpret_cast<const u32x4*>(w_rd + wb * L::kW + c * 2048 +
+                                                      16 * ((2 * gi + h) ^ w_swz));
+      W[c].w[0] = t[0], W[c].w[1] = t[1], W[c].w[2] = t[2], W[c].w[3] = t[3];
+    } else {
+      const u32x2* q = reinterpret_cast<const u32x2*>(w_rd + wb * L::kW + c * 1536);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) W[c].w[2 * i] = q[i][0], W[c].w[2 * i + 1] = q[i][1];
+    }
   };
   auto read_a = [&](int mb, int st, int buf) {
     A[st & 1][mb] = *reinterpret_cast<const bf16x8*>(a_rd + buf * kWideA + mb * 4096 +
                                                      16 * ((4 * h + st) ^ a_swz));
   };
-  // A(j + 1) has the next A stage and one W unit behind it in every stage, and
-  // the W unit and S block needed next are older: when no more than that is in
-  // flight they have landed, for this wave and, after the barrier, for all.
+  // A(j + 1) has the next A stage and one 4-bit W unit (or two 6-bit ones, 3
+  // loads each) behind it in every stage, and the W unit and S block needed
+  // next are older: when no more than that is in flight they have landed, for
+  // this wave and, after the barrier, for all.
   // (lgkmcnt: this wave's reads of the buffer that is given up have returned.)
   auto arrive = [&]() {
-    if constexpr (kAIns == 2)
-      asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kAIns + (BITS == 4 ? 4 : 6)) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
@@ -1082,8 +1113,8 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
   for (int c = 0; c < 2; ++c) read_s(c, 0), read_w(c, 0, 0);
 #pragma unroll
   for (int mb = 0; mb < NMB; ++mb) read_a(mb, 0, 0);
-  dequant_job<4>(W[0], S[0], 0, 0, B[0]);
-  dequant_job<4>(W[0], S[0], 0, 1, B[0]);
+  dequant_job<BITS>(W[0], S[0], 0, 0, B[0]);
+  dequant_job<BITS>(W[0], S[0], 0, 1, B[0]);
   int buf = 0;  // of stage j
   for (int j0 = 0; j0 < n_groups; j0 += 8) {
 #pragma unroll
@@ -1093,11 +1124,14 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
       const int un = (u + 1) & 7;  // the next group's scale entry
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        if (st == 1 && (u & 1)) {
-          // both groups of the unit are in registers (their last words were
-          // waited for in step 0): its buffer takes the unit after next, and
-          // after the first unit of a block, S's the block after next
-          load_w((j >> 1) + 2);
+        if (st == 1) {
+          // the unit's words are in registers (the last were waited for in
+          // step 0): its buffer takes the next unit not yet loaded; at the
+          // second group of a block, S's buffer the block after next
+          if (BITS == 6)
+            load_w(j + 3, buf);
+          else if (u & 1)
+            load_w((j >> 1) + 2, (u >> 1) & 1);
           if (u == 1) load_s((j0 >> 3) + 2);
         }
 #pragma unroll
@@ -1115,13 +1149,13 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
                 // and this stage's buffer takes the stage after the next two.
                 arrive();
                 load_a(j + 3, buf);
-                read_w(0, ((u + 1) >> 1) & 1, (u + 1) & 1);
+                read_w(0, BITS == 4 ? ((u + 1) >> 1) & 1 : nbuf, (u + 1) & 1);
                 if (u == 7) read_s(0, (j0 >> 3) + 1);
               }
               read_a(mb, 0, nbuf);
             }
             if (c == 1 && st == 3 && mb == 0) {
-              read_w(1, ((u + 1) >> 1) & 1, (u + 1) & 1);
+              read_w(1, BITS == 4 ? ((u + 1) >> 1) & 1 : nbuf, (u + 1) & 1);
               if (u == 7) read_s(1, (j0 >> 3) + 1);
             }
             // the operand of the next set or step (or stage), 4 values after
@@ -1129,11 +1163,11 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
 #pragma unroll
             for (int q = mb; q < (NMB == 1 ? 2 : mb < 2 ? mb + 1 : mb); ++q) {
               if (c == 0)
-                dequant_job<4>(W[1], S[1], u, 2 * st + q, B[1]);
+                dequant_job<BITS>(W[1], S[1], u, 2 * st + q, B[1]);
               else if (st < 3)
-                dequant_job<4>(W[0], S[0], u, 2 * st + 2 + q, B[0]);
+                dequant_job<BITS>(W[0], S[0], u, 2 * st + 2 + q, B[0]);
               else
-                dequant_job<4>(W[0], S[0], un, q, B[0]);
+                dequant_job<BITS>(W[0], S[0], un, q, B[0]);
             }
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -1147,22 +1181,24 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
   __syncthreads();
 }
 
+template <int BITS>
 __device__ __forceinline__ void gemm_wide_any(int nmb, int n_groups, const uint8_t* act,
                                               const int32_t* order, int kk, int cols, int p0,
                                               int m, const WideRows& wr, uint8_t* lds,
                                               f32x16 (&acc)[2][kMB]) {
   switch (nmb) {
-    case 1: gemm_tile_wide<1>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
-    case 2: gemm_tile_wide<2>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
-    case 3: gemm_tile_wide<3>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
-    default: gemm_tile_wide<4>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    case 1: gemm_tile_wide<BITS, 1>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    case 2: gemm_tile_wide<BITS, 2>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    case 3: gemm_tile_wide<BITS, 3>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
+    default: gemm_tile_wide<BITS, 4>(n_groups, act, order, kk, cols, p0, m, wr, lds, acc); break;
   }
 }
 
 // Wave w: gate rows (set 0) and up rows (set 1) of the same 32 columns, so
 // the SwiGLU needs no exchange.
+template <int BITS>
 __global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const PrefillArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kWideLds];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Wide<BITS>::kLds];
   TileInfo ti;
   int cb;
   if (!xcd_work<kTileM>(a, a.out_cols / kWideGuCols, ti, cb)) return;
@@ -1170,7 +1206,7 @@ __global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const PrefillA
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const uint8_t* base = a.slab + size_t(ti.slot) * size_t(a.expert_bytes);
-  const size_t row_bytes = size_t(a.cols) / 2;
+  const size_t row_bytes = size_t(a.cols) * BITS / 8;
   const int groups = a.cols / 64;
   const int col0 = cb * kWideGuCols + wave * 32;
   WideRows wr;
@@ -1182,7 +1218,7 @@ __global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const PrefillA
   wr.b[1] = uniform_ptr(base + a.b1 + size_t(col0) * groups * 2);
   f32x16 acc[2][kMB];
   const int nmb = __builtin_amdgcn_readfirstlane((ti.m + 31) >> 5);
-  gemm_wide_any(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), a.order, a.kk, a.cols, ti.p0,
+  gemm_wide_any<BITS>(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), a.order, a.kk, a.cols, ti.p0,
                 ti.m, wr, lds, acc);
   const int h = lane >> 5;
   uint16_t* hout = static_cast<uint16_t*>(a.out) + col0 + (lane & 31);
@@ -1197,8 +1233,9 @@ __global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const PrefillA
   }
 }
 
+template <int BITS>
 __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kWideLds];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Wide<BITS>::kLds];
   __shared__ int32_t s_ord[kTileM];
   TileInfo ti;
   int cb;
@@ -1216,7 +1253,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
     return;
   }
   const uint8_t* base = a.slab + size_t(ti.slot) * size_t(a.expert_bytes);
-  const size_t row_bytes = size_t(a.cols) / 2;
+  const size_t row_bytes = size_t(a.cols) * BITS / 8;
   const int groups = a.cols / 64;
   const int col0 = cb * kWideDnCols + wave * 64;
   WideRows wr;
@@ -1229,7 +1266,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
   if (int(threadIdx.x) < ti.m) s_ord[threadIdx.x] = a.order[ti.p0 + threadIdx.x];
   f32x16 acc[2][kMB];
   const int nmb = __builtin_amdgcn_readfirstlane((ti.m + 31) >> 5);
-  gemm_wide_any(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), nullptr, 1, a.cols, ti.p0,
+  gemm_wide_any<BITS>(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), nullptr, 1, a.cols, ti.p0,
                 ti.m, wr, lds, acc);
   const int h = lane >> 5;
   if (a.out_f32 || !a.out_vec) {
@@ -1253,7 +1290,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
   // bf16 rows go out through LDS as 16-byte pieces, as in down_mfma_kernel
   constexpr int kEp = kWideDnCols + 8;
   constexpr int kPieces = kWideDnCols / 8;
-  static_assert(kTileM * kEp * 2 <= kWideLds, "output tile in LDS");
+  static_assert(kTileM * kEp * 2 <= Wide<BITS>::kLds, "output tile in LDS");
   uint16_t* ot = reinterpret_cast<uint16_t*>(lds);
 #pragma unroll
   for (int c = 0; c < 2; ++c)
@@ -1306,13 +1343,14 @@ bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids) {
   return rows >= 1024 && rows >= 16L * n_ids;
 }
 
-// The wide 128-row form (4-bit) once the narrow one's gate/up items, 128
-// columns each, are more than one a CU: below that a launch takes one block's
-// time, and the narrow block's is shorter.  Measured us a layer, narrow / wide:
-// hidden 1024, 32 experts 1400 tokens 67 / 78, 2000 tokens 98 / 81, 16000
-// tokens 411 / 366; Qwen3-235B shapes 520 tokens 491 / 492, 2048 tokens
-// 1044 / 967, 8192 tokens 3346 / 2851; DeepSeek-V3 shapes 2048 tokens
-// 3717 / 3372.  Tiles are estimated as full ones plus half of one an expert.
+// The wide 128-row form once the narrow one's gate/up items, 128 columns each,
+// are more than one a CU: below that a launch takes one block's time, and the
+// narrow block's is shorter.  Measured us a layer, narrow / wide: hidden 1024,
+// 32 experts 1400 tokens 67 / 78, 2000 tokens 98 / 81, 16000 tokens 411 / 366;
+// Qwen3-235B shapes 520 tokens 491 / 492, 2048 tokens 1044 / 967, 8192 tokens
+// 3346 / 2851; DeepSeek-V3 shapes 2048 tokens 3717 / 3372; Qwen3-Next shapes
+// (6-bit) 1500 tokens 672 / 574, 5000 tokens 1004 / 883, 16000 tokens 2760 /
+// 2308.  Tiles are estimated as full ones plus half of one an expert.
 // PMOE_PREFILL_WIDE=1 / 0 pins either (same outputs).
 bool prefill_wide(const pmoe_geom* g, int n, int kk, int n_experts) {
   const char* v = getenv("PMOE_PREFILL_WIDE");
@@ -1356,11 +1394,14 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
   {
     const int items = g->inter / kGuCols * max_tiles;
     dim3 grid((items + 7) / 8 * 8);  // a multiple of 8: xcd_work deals items per XCD
+    dim3 wide_grid((g->inter / kWideGuCols * max_tiles + 7) / 8 * 8);
     ProfScope prof_scope(K_PREFILL_GATEUP, st);
     if (g->bits == 4 && small)
       gateup_mfma_kernel<4, 1><<<grid, kThreads, 0, st>>>(a);
     else if (g->bits == 4 && wide)
-      gateup_wide_kernel<<<(g->inter / kWideGuCols * max_tiles + 7) / 8 * 8, kThreads, 0, st>>>(a);
+      gateup_wide_kernel<4><<<wide_grid, kThreads, 0, st>>>(a);
+    else if (wide && !small)
+      gateup_wide_kernel<6><<<wide_grid, kThreads, 0, st>>>(a);
     else if (g->bits == 4)
       gateup_mfma_kernel<4, kMB><<<grid, kThreads, 0, st>>>(a);
     else if (small)
@@ -1383,11 +1424,14 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
   {
     const int items = g->hidden / kDnCols * max_tiles;
     dim3 grid((items + 7) / 8 * 8);
+    dim3 wide_grid((g->hidden / kWideDnCols * max_tiles + 7) / 8 * 8);
     ProfScope prof_scope(K_PREFILL_DOWN, st);
     if (g->bits == 4 && small)
       down_mfma_kernel<4, 1><<<grid, kThreads, 0, st>>>(a);
     else if (g->bits == 4 && wide)
-      down_wide_kernel<<<(g->hidden / kWideDnCols * max_tiles + 7) / 8 * 8, kThreads, 0, st>>>(a);
+      down_wide_kernel<4><<<wide_grid, kThreads, 0, st>>>(a);
+    else if (wide && !small)
+      down_wide_kernel<6><<<wide_grid, kThreads, 0, st>>>(a);
     else if (g->bits == 4)
       down_mfma_kernel<4, kMB><<<grid, kThreads, 0, st>>>(a);
     else if (small)

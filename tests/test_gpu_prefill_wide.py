@@ -20,13 +20,14 @@ DEV = "cuda"
 COUNTS = [300, 129, 128, 127, 97, 96, 1, 31, 32, 33, 64, 65, 90]
 
 
-@pytest.mark.parametrize("hidden,inter", [(1024, 512), (2048, 1536), (512, 1024), (4096, 512)])
-def test_wide_matches_narrow_and_oracle(hidden, inter, monkeypatch):
+@pytest.mark.parametrize("hidden,inter,bits", [(1024, 512, 4), (2048, 1536, 4), (512, 1024, 4),
+                                               (4096, 512, 4), (1024, 512, 6), (2048, 1536, 6)])
+def test_wide_matches_narrow_and_oracle(hidden, inter, bits, monkeypatch):
     from pagedmoe_amd import kernels as K
     monkeypatch.setenv("PMOE_STREAM", "0")
     monkeypatch.setenv("PMOE_PREFILL_SMALL", "0")
     n, k, e = 330, 4, len(COUNTS)
-    g, slab, experts = _setup(hidden, inter, 4, e, 60)
+    g, slab, experts = _setup(hidden, inter, bits, e, 60)
     rng = np.random.default_rng(hidden + inter)
     xb = O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32))
     ids = _ids(COUNTS, k, rng, n)
@@ -42,7 +43,7 @@ def test_wide_matches_narrow_and_oracle(hidden, inter, monkeypatch):
     gone = (ids < 0) | (ids == 12)
     assert (y[gone] == 0).all()
     ref = O.switch_glu_f64(xb, np.where(gone, 0, ids), experts)
-    check_close(y[~gone], ref[~gone], f"wide {hidden}x{inter}")
+    check_close(y[~gone], ref[~gone], f"wide {hidden}x{inter} {bits}-bit")
     # unaligned output rows take the element-wise stores
     big = torch.full((n * k * hidden + 8,), float("nan"), dtype=torch.bfloat16, device=DEV)
     un = big[1:1 + n * k * hidden]
