@@ -1125,13 +1125,18 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         if (st == 1) {
-          // the unit's words are in registers (the last were waited for in
-          // step 0): its buffer takes the next unit not yet loaded; at the
-          // second group of a block, S's buffer the block after next
-          if (BITS == 6)
+          // the unit's words are in registers: its buffer takes the next unit
+          // not yet loaded; at the second group of a block, S's buffer the
+          // block after next.  4-bit: set 1's words are one 16-byte read, and
+          // step 0 dequantized from it.  6-bit: three reads, and step 0 uses
+          // the first alone, so the others are waited for here (with step 1's
+          // fragments, which its MFMAs need at once).
+          if (BITS == 6) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             load_w(j + 3, buf);
-          else if (u & 1)
+          } else if (u & 1) {
             load_w((j >> 1) + 2, (u >> 1) & 1);
+          }
           if (u == 1) load_s((j0 >> 3) + 2);
         }
 #pragma unroll

@@ -21,7 +21,8 @@ COUNTS = [300, 129, 128, 127, 97, 96, 1, 31, 32, 33, 64, 65, 90]
 
 
 @pytest.mark.parametrize("hidden,inter,bits", [(1024, 512, 4), (2048, 1536, 4), (512, 1024, 4),
-                                               (4096, 512, 4), (1024, 512, 6), (2048, 1536, 6)])
+                                               (4096, 512, 4), (1024, 512, 6), (2048, 1536, 6),
+                                               (4096, 1024, 6)])
 def test_wide_matches_narrow_and_oracle(hidden, inter, bits, monkeypatch):
     from pagedmoe_amd import kernels as K
     monkeypatch.setenv("PMOE_STREAM", "0")
