@@ -152,6 +152,14 @@ size_t pmoe_moe_workspace(const pmoe_geom* g, int n, int k, int shared,
  * that reason about tile edges. */
 int pmoe_prefill_tile_rows(int n, int kk, int n_experts);
 
+/* 1 when the prefill expert GEMMs of such a call (slab and x as passed to it)
+ * run in the wide 128-row form, 0 in another: one round of tiles or fewer,
+ * 32-row tiles, or a slab, component offset or x that is not 16-byte aligned.
+ * The outputs are the same either way; PMOE_PREFILL_WIDE=1 / 0 pins it where
+ * it can run.  No reference counterpart. */
+int pmoe_prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n, int kk,
+                      int n_experts);
+
 /* 1 when the experts of n tokens with kk columns (shared: the last is a
  * shared expert's) run as streamed 16-column tiles: between the decode GEMV
  * (few rows an expert) and the prefill GEMMs (more than 32 rows an expert on

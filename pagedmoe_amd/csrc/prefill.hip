@@ -1356,8 +1356,21 @@ bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids) {
 // 3346 / 2851; DeepSeek-V3 shapes 2048 tokens 3717 / 3372; Qwen3-Next shapes
 // (6-bit) 1500 tokens 672 / 574, 5000 tokens 1004 / 883, 16000 tokens 2760 /
 // 2308.  Tiles are estimated as full ones plus half of one an expert.
-// PMOE_PREFILL_WIDE=1 / 0 pins either (same outputs).
-bool prefill_wide(const pmoe_geom* g, int n, int kk, int n_experts) {
+// PMOE_PREFILL_WIDE=1 / 0 pins either (same outputs) where the wide form can run.
+//
+// It moves 16 bytes a lane from the activations and the weights straight into
+// LDS, so all of them have to lie on 16 bytes (rows do: both dims are multiples
+// of 512).  The narrow form loads through registers and takes any pointer.
+bool wide_layout(const pmoe_geom* g, const void* slab, const void* x) {
+  uintptr_t at = reinterpret_cast<uintptr_t>(slab) | reinterpret_cast<uintptr_t>(x) |
+                 uintptr_t(g->expert_bytes);
+  for (int c = 0; c < PMOE_NCOMP; ++c) at |= uintptr_t(g->off[c]);
+  return at % 16 == 0;
+}
+
+bool prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n, int kk,
+                  int n_experts) {
+  if (!wide_layout(g, slab, x)) return false;
   const char* v = getenv("PMOE_PREFILL_WIDE");
   if (v && (v[0] == '0' || v[0] == '1')) return v[0] == '1';
   const long tiles = long(n) * kk / kTileM + n_experts / 2;
@@ -1376,7 +1389,9 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
                    int64_t(n) * kk * g->inter < (int64_t(1) << 31),
                "prefill: activations exceed 2^31 elements");
   const bool small = tile_m == 32;
-  const bool wide = prefill_wide(g, n, kk, n_experts);
+  // (h is carved from the workspace, as aligned as its base)
+  const bool wide = reinterpret_cast<uintptr_t>(h) % 16 == 0 &&
+                    prefill_wide(g, slab, x, n, kk, n_experts);
   PrefillArgs a{};
   a.slab = slab;
   a.expert_bytes = g->expert_bytes;
@@ -1449,3 +1464,12 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
 }
 
 }  // namespace pmoe
+
+extern "C" int pmoe_prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n,
+                                 int kk, int n_experts) {
+  if (!g || n <= 0 || kk <= 0 || n_experts <= 0) return 0;
+  return pmoe::prefill_tile_rows(n, kk, n_experts) == pmoe::kTileM &&
+                 pmoe::prefill_wide(g, slab, x, n, kk, n_experts)
+             ? 1
+             : 0;
+}

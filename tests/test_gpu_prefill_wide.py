@@ -17,6 +17,13 @@ from tests.util import bits_to_bf16_tensor, check_close
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
+
+
+def _wide(g, slab, x, n, k, e):
+    from pagedmoe_amd._lib import lib
+    return lib().pmoe_prefill_wide(ctypes.byref(g), slab.data_ptr, x.data_ptr(), n, k, e)
+
+
 COUNTS = [300, 129, 128, 127, 97, 96, 1, 31, 32, 33, 64, 65, 90]
 
 
@@ -38,6 +45,7 @@ def test_wide_matches_narrow_and_oracle(hidden, inter, bits, monkeypatch):
     got = []
     for pin in ("0", "1"):
         monkeypatch.setenv("PMOE_PREFILL_WIDE", pin)
+        assert _wide(g, slab, x, n, k, e) == int(pin)
         got.append(K.switch_glu(g, slab.buf, table, e, x, inds))
     assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
     y = got[1].float().cpu().numpy()
@@ -56,6 +64,29 @@ def test_wide_matches_narrow_and_oracle(hidden, inter, bits, monkeypatch):
     torch.cuda.synchronize()
     assert torch.equal(got[1].reshape(-1).view(torch.int16), un.view(torch.int16))
     assert torch.isnan(big[0]) and torch.isnan(big[-7:]).all()
+    slab.release()
+
+
+@pytest.mark.parametrize("bits", [4, 6])
+def test_unaligned_activations(bits, monkeypatch):
+    """x at a 2-byte offset (the narrow form) gives the aligned call's bits."""
+    from pagedmoe_amd import kernels as K
+    monkeypatch.setenv("PMOE_STREAM", "0")
+    monkeypatch.setenv("PMOE_PREFILL_SMALL", "0")
+    monkeypatch.setenv("PMOE_PREFILL_WIDE", "1")
+    n, k, e, hidden = 330, 4, len(COUNTS), 1024
+    g, slab, _ = _setup(hidden, 512, bits, e, 63)
+    rng = np.random.default_rng(64)
+    xb = O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32))
+    inds = torch.from_numpy(_ids(COUNTS, k, rng, n)).to(DEV)
+    table = torch.arange(e, dtype=torch.int32, device=DEV)
+    x = bits_to_bf16_tensor(xb, DEV)
+    un = torch.empty(n * hidden + 8, dtype=torch.bfloat16, device=DEV)[1:1 + n * hidden]
+    un = un.view(n, hidden).copy_(x)
+    assert x.data_ptr() % 16 == 0 and un.data_ptr() % 16 == 2
+    assert _wide(g, slab, x, n, k, e) == 1 and _wide(g, slab, un, n, k, e) == 0
+    y, yu = (K.switch_glu(g, slab.buf, table, e, t, inds) for t in (x, un))
+    assert torch.equal(y.view(torch.int16), yu.view(torch.int16))
     slab.release()
 
 
