@@ -154,7 +154,8 @@ int pmoe_prefill_tile_rows(int n, int kk, int n_experts);
 
 /* 1 when the prefill expert GEMMs of such a call (slab and x as passed to it)
  * run in the wide 128-row form, 0 in another: one round of tiles or fewer,
- * 32-row tiles, or a slab, component offset or x that is not 16-byte aligned.
+ * 32-row tiles, a slab, component offset or x that is not 16-byte aligned, or
+ * an up component before its gate one (or 2 GiB behind it).
  * The outputs are the same either way; PMOE_PREFILL_WIDE=1 / 0 pins it where
  * it can run.  No reference counterpart. */
 int pmoe_prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n, int kk,

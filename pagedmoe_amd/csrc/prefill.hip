@@ -1361,10 +1361,17 @@ bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids) {
 // It moves 16 bytes a lane from the activations and the weights straight into
 // LDS, so all of them have to lie on 16 bytes (rows do: both dims are multiples
 // of 512).  The narrow form loads through registers and takes any pointer.
+// A gate/up wave addresses its up rows by an unsigned 32-bit offset from its
+// gate rows, so each up component has to follow its gate one by less than
+// 2 GiB (31 rows and a chunk are added).
 bool wide_layout(const pmoe_geom* g, const void* slab, const void* x) {
   uintptr_t at = reinterpret_cast<uintptr_t>(slab) | reinterpret_cast<uintptr_t>(x) |
                  uintptr_t(g->expert_bytes);
   for (int c = 0; c < PMOE_NCOMP; ++c) at |= uintptr_t(g->off[c]);
+  for (int c = PMOE_GATE_W; c <= PMOE_GATE_B; ++c) {
+    const int64_t up = g->off[c + PMOE_UP_W] - g->off[c];
+    if (up < 0 || up >= (int64_t(1) << 31)) return false;
+  }
   return at % 16 == 0;
 }
 

@@ -90,6 +90,36 @@ def test_unaligned_activations(bits, monkeypatch):
     slab.release()
 
 
+@pytest.mark.parametrize("bits", [4, 6])
+def test_components_in_another_order(bits, monkeypatch):
+    """Slots whose components lie in the reverse order (down first, gate last):
+    the bits of the usual layout."""
+    from pagedmoe_amd import kernels as K
+    from pagedmoe_amd._lib import geom
+    monkeypatch.setenv("PMOE_STREAM", "0")
+    monkeypatch.setenv("PMOE_PREFILL_SMALL", "0")
+    monkeypatch.setenv("PMOE_PREFILL_WIDE", "1")
+    n, k, e, hidden = 330, 4, len(COUNTS), 1024
+    g, slab, _ = _setup(hidden, 512, bits, e, 65)
+    r, at = geom(hidden, 512, bits), 0
+    for c in reversed(range(9)):
+        r.off[c] = at
+        at += -(-g.nbytes[c] // 256) * 256
+    src = slab.buf.view(e, g.expert_bytes)
+    dst = torch.empty_like(src)
+    for c in range(9):
+        dst[:, r.off[c]:r.off[c] + g.nbytes[c]] = src[:, g.off[c]:g.off[c] + g.nbytes[c]]
+    rng = np.random.default_rng(66)
+    x = bits_to_bf16_tensor(O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32)), DEV)
+    inds = torch.from_numpy(_ids(COUNTS, k, rng, n)).to(DEV)
+    table = torch.arange(e, dtype=torch.int32, device=DEV)
+    assert _wide(g, slab, x, n, k, e) == 1 and _wide(r, slab, x, n, k, e) == 0
+    y = K.switch_glu(g, slab.buf, table, e, x, inds)
+    yr = K.switch_glu(r, dst.view(-1), table, e, x, inds)
+    assert torch.equal(y.view(torch.int16), yr.view(torch.int16))
+    slab.release()
+
+
 def test_wide_block_in_a_graph(monkeypatch):
     """The whole block in the wide form, replayed from a HIP graph."""
     from pagedmoe_amd import kernels as K

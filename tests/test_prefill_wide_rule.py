@@ -40,6 +40,17 @@ def test_unaligned_operands_keep_the_narrow_form(bits, pin, monkeypatch):
     assert wide(h) == 0
 
 
+@pytest.mark.parametrize("bits", [4, 6])
+@pytest.mark.parametrize("comp", [0, 1, 2])
+def test_up_component_before_its_gate_keeps_the_narrow_form(bits, comp):
+    g = geom(4096, 1536, bits)
+    g.off[comp], g.off[comp + 3] = g.off[comp + 3], g.off[comp]
+    assert wide(g) == 0
+    g = geom(4096, 1536, bits)
+    g.off[comp + 3] = g.off[comp] + (1 << 31)
+    assert wide(g) == 0
+
+
 def test_pins_and_tile_height(monkeypatch):
     g = geom(4096, 1536, 4)
     assert wide(g, n=512) == 0  # 32-row tiles
