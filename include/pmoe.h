@@ -164,8 +164,10 @@ int pmoe_prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n
 /* 1 when the experts of n tokens with kk columns (shared: the last is a
  * shared expert's) run as streamed 16-column tiles: between the decode GEMV
  * (few rows an expert) and the prefill GEMMs (more than 32 rows an expert on
- * average); PMOE_STREAM=1 / 0 pins it where the shape is covered.  No
- * reference counterpart. */
+ * average); PMOE_STREAM=1 / 0 pins it where the shape is covered.  Slots whose
+ * components do not all lie inside a stride below 2 GiB, on 4-byte offsets,
+ * are not (nor is a slab that is not 4-byte aligned).  No reference
+ * counterpart. */
 int pmoe_stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int shared);
 
 /* A MoE workspace starts with a 1,352,960-byte synchronisation header (grid

@@ -237,8 +237,9 @@ int check_route_cfg(const pmoe_route_cfg* rc) {
 //     40 tokens 61 / 54).
 // PMOE_STREAM=1 / 0 pins the form where it covers the shape (read per call, so
 // the two can be compared).
-bool stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int n_ids) {
-  if (!stream_covers(g)) return false;
+bool stream_wanted(const pmoe_geom* g, const uint8_t* slab, int n, int kk, int n_experts,
+                   int n_ids) {
+  if (!stream_covers(g, slab)) return false;
   const char* v = getenv("PMOE_STREAM");
   if (v && (v[0] == '0' || v[0] == '1')) return v[0] == '1';
   const long rows = long(n) * kk;
@@ -258,7 +259,7 @@ int run_experts(const pmoe_geom* g, const uint8_t* slab, const int32_t* table, i
                 int max_rows_per_expert, const MoeWs& w, void* y, int y_f32, hipStream_t st) {
   const int rows = n * kk;
   const int n_ids = n_experts + (kk > k ? 1 : 0);
-  const bool stream = stream_wanted(g, n, kk, n_experts, n_ids);
+  const bool stream = stream_wanted(g, slab, n, kk, n_experts, n_ids);
   const bool prefill = !stream && prefill_wanted(g, n, kk, n_ids);
   const int tm = stream ? stream_tile_rows() : prefill ? prefill_tile_rows(n, kk, n_experts) : 0;
   // the tile list carries the slots of this table
@@ -401,7 +402,7 @@ int decode_block(const pmoe_geom* g, const pmoe_route_cfg* rc, const uint8_t* sl
   }
   // streamed experts into fp32 per-slot rows (a pinned decode form compares
   // the GEMV paths and keeps them)
-  if (n > 1 && !getenv("PMOE_DECODE_FUSED") && stream_wanted(g, n, kk, e, e + shared)) {
+  if (n > 1 && !getenv("PMOE_DECODE_FUSED") && stream_wanted(g, slab, n, kk, e, e + shared)) {
     // Up to 12 tokens the router launch's last block routes, one token a wave
     // and round; beyond, its rounds cost more than a routing launch with a wave
     // for every token (us a layer, last block / launch: Qwen3-235B shapes 12
@@ -493,7 +494,7 @@ using pmoe::MoeWs;
 
 extern "C" int pmoe_stream_wanted(const pmoe_geom* g, int n, int kk, int n_experts, int shared) {
   if (!g || n <= 0 || kk <= 0 || n_experts <= 0) return 0;
-  return pmoe::stream_wanted(g, n, kk, n_experts, n_experts + (shared ? 1 : 0)) ? 1 : 0;
+  return pmoe::stream_wanted(g, nullptr, n, kk, n_experts, n_experts + (shared ? 1 : 0)) ? 1 : 0;
 }
 
 extern "C" size_t pmoe_moe_workspace(const pmoe_geom* g, int n, int k, int shared,

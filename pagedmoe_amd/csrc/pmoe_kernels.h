@@ -202,7 +202,7 @@ int route_sigmoid(const float* logits, const float* bias, int n, int e, int n_gr
 // Experts of few rows each over the dispatch's tiles of stream_tile_rows()
 // rows (stream.hip): gate/up into h, down into y [rows, hidden] (fp32 when
 // y_f32, else bf16).
-bool stream_covers(const pmoe_geom* g);
+bool stream_covers(const pmoe_geom* g, const void* slab);
 int stream_tile_rows();
 int stream_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                    const int32_t* order, const int4* tiles, const int32_t* n_tiles, uint16_t* h,

@@ -498,16 +498,28 @@ int launch_stream(const StreamArgs& a, hipStream_t st) {
 
 int stream_tile_rows() { return kStreamRows; }
 
-bool stream_covers(const pmoe_geom* g) {
+// Shapes with a cut for both reductions, in slots that the buffer loads can
+// address: a resource spans one slot (32-bit offsets; what lies outside reads
+// as zero), so every component has to lie inside the slot's stride, on whole
+// words.
+bool stream_covers(const pmoe_geom* g, const void* slab) {
   const Cut gu = stream_cut(g->hidden), dn = stream_cut(g->inter);
-  return gu.g && dn.g && (g->bits == 4 || (gu.g <= 8 && dn.g <= 8));
+  if (!gu.g || !dn.g || (g->bits == 6 && (gu.g > 8 || dn.g > 8))) return false;
+  if (g->expert_bytes >= (int64_t(1) << 31)) return false;
+  uintptr_t at = reinterpret_cast<uintptr_t>(slab) | uintptr_t(g->expert_bytes);
+  const int64_t vals = int64_t(g->hidden) * g->inter;
+  for (int c = 0; c < PMOE_NCOMP; ++c) {
+    const int64_t bytes = c % 3 ? vals / 64 * 2 : vals * g->bits / 8;
+    if (g->off[c] < 0 || g->off[c] + bytes > g->expert_bytes) return false;
+    at |= uintptr_t(g->off[c]);
+  }
+  return at % 4 == 0;
 }
 
 int stream_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                    const int32_t* order, const int4* tiles, const int32_t* n_tiles, uint16_t* h,
                    void* y, int y_f32, hipStream_t st) {
-  PMOE_REQUIRE(stream_covers(g) && g->expert_bytes < (int64_t(1) << 31),
-               "stream: unsupported shape");
+  PMOE_REQUIRE(stream_covers(g, slab), "stream: unsupported shape");
   StreamArgs a{};
   a.slab = slab;
   a.expert_bytes = g->expert_bytes;

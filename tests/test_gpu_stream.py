@@ -97,6 +97,38 @@ def test_stream_unaligned_output_matches_aligned(monkeypatch):
     slab.release()
 
 
+@pytest.mark.parametrize("bits", [4, 6])
+def test_stream_components_in_arrays_of_their_own(bits, monkeypatch):
+    """A slab of one array a component over all experts (components beyond the
+    slot's stride) gives what the usual layout gives on the same path."""
+    from pagedmoe_amd import kernels as K
+    from pagedmoe_amd._lib import geom
+    n, k, e, hidden = 37, 2, 4, 1024
+    g, slab, _ = _setup(hidden, 512, bits, e, 92)
+    src = slab.buf.view(e, g.expert_bytes)
+    r, at = geom(hidden, 512, bits), 0
+    # every expert's gate weights, then every expert's up weights, ...: the
+    # stride of the largest component serves all
+    r.expert_bytes = max(g.nbytes)
+    dst = torch.empty(9 * e * r.expert_bytes, dtype=torch.uint8, device=DEV)
+    for c in range(9):
+        r.off[c] = at
+        rows = dst[at:at + e * r.expert_bytes].view(e, r.expert_bytes)
+        rows[:, :g.nbytes[c]] = src[:, g.off[c]:g.off[c] + g.nbytes[c]]
+        at += e * r.expert_bytes
+    rng = np.random.default_rng(93)
+    x = bits_to_bf16_tensor(O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32)), DEV)
+    inds = torch.from_numpy(np.stack([rng.choice(e, k, replace=False) for _ in range(n)])
+                            .astype(np.int32)).to(DEV)
+    table = torch.arange(e, dtype=torch.int32, device=DEV)
+    monkeypatch.setenv("PMOE_STREAM", "0")
+    y = K.switch_glu(g, slab.buf, table, e, x, inds)
+    monkeypatch.setenv("PMOE_STREAM", "1")
+    yr = K.switch_glu(r, dst, table, e, x, inds)
+    assert torch.equal(y.view(torch.int16), yr.view(torch.int16))
+    slab.release()
+
+
 @pytest.mark.parametrize("bits,n", [(4, 2), (4, 12), (4, 13), (4, 17), (6, 50)])
 def test_stream_block_vs_oracle(bits, n, monkeypatch):
     """The whole block with a gated shared expert (its rows are every token:

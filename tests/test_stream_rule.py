@@ -23,3 +23,28 @@ def test_stream_rule(hidden, inter, bits, e, kk, form, monkeypatch):
     shared = 1 if kk in (9, 11) else 0
     for n, want in form.items():
         assert lib().pmoe_stream_wanted(ctypes.byref(g), n, kk, e, shared) == want, n
+
+
+@pytest.mark.parametrize("bits", [4, 6])
+@pytest.mark.parametrize("pin", [None, "1"])
+def test_slots_the_buffer_loads_cannot_address(bits, pin, monkeypatch):
+    """A resource spans one slot: components outside the stride (one array a
+    component over all experts), strides of 2 GiB and offsets that are not
+    whole words stay on the general paths."""
+    from pagedmoe_amd._lib import geom, lib
+    monkeypatch.delenv("PMOE_STREAM", raising=False)
+    if pin:
+        monkeypatch.setenv("PMOE_STREAM", pin)
+
+    def wanted(edit):
+        g = geom(4096, 1024, bits)
+        edit(g)
+        return lib().pmoe_stream_wanted(ctypes.byref(g), 64, 8, 128, 0)
+
+    assert wanted(lambda g: None) == 1
+    for c in range(9):
+        assert wanted(lambda g: g.off.__setitem__(c, g.expert_bytes - g.nbytes[c] + 4)) == 0
+        assert wanted(lambda g: g.off.__setitem__(c, -256)) == 0
+        assert wanted(lambda g: g.off.__setitem__(c, g.off[c] + 2)) == 0
+    assert wanted(lambda g: setattr(g, "expert_bytes", 1 << 31)) == 0
+    assert wanted(lambda g: setattr(g, "expert_bytes", (1 << 31) - 256)) == 1
