@@ -134,6 +134,17 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
   }
 }
 
+// A launch holds at most 2^32 - 1 threads, 8 to a group: longer arrays go out
+// in several.  go(first group, groups, blocks).
+template <class Go>
+void each_launch(size_t groups, Go go) {
+  constexpr size_t kMost = size_t(1) << 28;
+  for (size_t g0 = 0; g0 < groups; g0 += kMost) {
+    const size_t n = groups - g0 < kMost ? groups - g0 : kMost;
+    go(g0, n, unsigned((n + 31) / 32));
+  }
+}
+
 }  // namespace
 
 int quantize(const float* w, int rows, int cols, int bits, int group, uint32_t* q,
@@ -144,9 +155,13 @@ int quantize(const float* w, int rows, int cols, int bits, int group, uint32_t* 
   PMOE_REQUIRE(rows >= 0 && cols > 0 && cols % 64 == 0, "quantize: cols must be a multiple of 64");
   const size_t n = size_t(rows) * (cols / 64);
   if (n == 0) return PMOE_OK;
-  const unsigned blocks = unsigned((n + 31) / 32);
   const bool vec = reinterpret_cast<uintptr_t>(w) % 16 == 0;
-  auto go = [&](auto kernel) { kernel<<<blocks, 256, 0, st>>>(w, n, q, scales, biases); };
+  auto go = [&](auto kernel) {
+    each_launch(n, [&](size_t g0, size_t groups, unsigned blocks) {
+      kernel<<<blocks, 256, 0, st>>>(w + g0 * 64, groups, q + g0 * (2 * bits), scales + g0,
+                                     biases + g0);
+    });
+  };
   if (bits == 4)
     vec ? go(quantize_kernel<4, true>) : go(quantize_kernel<4, false>);
   else
@@ -163,9 +178,13 @@ int dequant(const uint32_t* q, const uint16_t* scales, const uint16_t* biases, i
   PMOE_REQUIRE(rows >= 0 && cols > 0 && cols % 64 == 0, "dequant: cols must be a multiple of 64");
   const size_t n = size_t(rows) * (cols / 64);
   if (n == 0) return PMOE_OK;
-  const unsigned blocks = unsigned((n + 31) / 32);
   const bool vec = reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  auto go = [&](auto kernel) { kernel<<<blocks, 256, 0, st>>>(q, scales, biases, n, out); };
+  auto go = [&](auto kernel) {
+    each_launch(n, [&](size_t g0, size_t groups, unsigned blocks) {
+      kernel<<<blocks, 256, 0, st>>>(q + g0 * (2 * bits), scales + g0, biases + g0, groups,
+                                     out + g0 * 64);
+    });
+  };
   if (bits == 4)
     vec ? go(dequant_kernel<4, true>) : go(dequant_kernel<4, false>);
   else

@@ -63,3 +63,26 @@ def test_dequant_unaligned_output(bits):
     assert torch.equal(big[1:1 + rows * cols],
                        K.dequant(q, s, b, bits).view(torch.int16).reshape(-1))
     assert int(big[0]) == -1 and bool((big[1 + rows * cols:] == -1).all())
+
+
+def test_more_threads_than_one_launch_holds():
+    """2^29 + 40 groups (8 lanes each: over 2^32 threads), 88 GB: the groups
+    around each launch's first and last against the same groups alone."""
+    from pagedmoe_amd import kernels as K
+    cols, rows = 512, (1 << 26) + 5
+    if torch.cuda.mem_get_info()[0] < 110e9:
+        pytest.skip("needs 88 GB")
+    per = cols // 64
+    q = torch.empty((rows, cols // 8), dtype=torch.int32, device=DEV)
+    s, b = (torch.empty((rows, per), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    w = torch.from_numpy(_values("normal", (16, cols), np.random.default_rng(6))).to(DEV)
+    seams = [slice(0, 16), slice((1 << 25) - 8, (1 << 25) + 8), slice((1 << 26) - 11, rows)]
+    for at in seams:
+        q[at], s[at], b[at] = K.quantize(w, 4)
+    out = K.dequant(q, s, b, 4)
+    for at in seams:
+        assert torch.equal(out[at].view(torch.int16),
+                           K.dequant(q[at].clone(), s[at].clone(), b[at].clone(), 4)
+                           .view(torch.int16))
+    del q, s, b, out
+    torch.cuda.empty_cache()
