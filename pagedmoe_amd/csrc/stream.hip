@@ -264,6 +264,13 @@ __device__ __forceinline__ void tile_mfma(WTile<BITS, G>& t, const XTile<G> (&x)
   }
 }
 
+// z, or NaN where v holds an infinity or a NaN.
+__device__ __forceinline__ float finite_or_nan(const f32x4& v, float z) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) z = __builtin_fmaf(v[i], 0.0f, z);
+  return z;
+}
+
 // A block's current tile.
 struct Seg {
   __amdgpu_buffer_rsrc_t slot;  // the expert's weights
@@ -293,7 +300,7 @@ struct StreamKernel {
   template <int MT>
   static __device__ __forceinline__ void run(const StreamArgs& a, const Seg& sg, int r0, int st0,
                                              int st1, float* part, int& buf,
-                                             const int32_t* s_row) {
+                                             const int32_t* s_row, uint32_t* s_odd) {
     constexpr int E = ring<MT>();
     const int lane = threadIdx.x & 63;
     const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -362,6 +369,7 @@ struct StreamKernel {
       constexpr int kQuads = kStepCols / 4;
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));  // opaque: addresses recomputed here, not held across the loop
+      float odd = 0.0f;  // NaN once an output is infinite or NaN (redo_range)
       for (int i = tid; i < MT * 16 * kQuads; i += kThreads) {
         const int c4 = i % kQuads, j = i / kQuads;
         const int mt = j >> 4;
@@ -372,11 +380,16 @@ struct StreamKernel {
         f32x4 v = *reinterpret_cast<const f32x4*>(q);
 #pragma unroll
         for (int sl = 1; sl < NSL; ++sl) v += *reinterpret_cast<const f32x4*>(q + sl * kPart);
+        odd = finite_or_nan(v, DUAL ? 0.0f : odd);
         if constexpr (DUAL) {
+          // Branched on between the two sums, not once after the loop: with
+          // both sums' reads in flight the longest slices spill.
+          if (odd != 0.0f) *s_odd = 1;
           f32x4 u = *reinterpret_cast<const f32x4*>(q + kTilePart);
 #pragma unroll
           for (int sl = 1; sl < NSL; ++sl)
             u += *reinterpret_cast<const f32x4*>(q + kTilePart + sl * kPart);
+          if (finite_or_nan(u, 0.0f) != 0.0f) *s_odd = 1;
 #pragma unroll
           for (int c = 0; c < 4; ++c) v[c] = silu_fast(v[c]) * u[c];
         }
@@ -395,10 +408,108 @@ struct StreamKernel {
           }
         }
       }
+      if (!DUAL && odd != 0.0f) *s_odd = 1;
       buf ^= 1;
     }
   }
 };
+
+// One weight row times one activation row, group by group: lanes take a group
+// each, weights dequantized before the product.
+template <int BITS>
+__device__ __forceinline__ float plain_dot(const uint32_t* w, const uint16_t* s, const uint16_t* b,
+                                           const uint16_t* x, int groups) {
+  float p = 0.0f;
+  for (int g = threadIdx.x & 63; g < groups; g += 64) {
+    const float sg = bf16f(s[g]), bg = bf16f(b[g]);
+    uint64_t bits = 0;
+    int have = 0, wi = g * (2 * BITS);
+#pragma unroll 1
+    for (int k = 0; k < 64; ++k) {
+      if (have < BITS) bits |= uint64_t(w[wi++]) << have, have += 32;
+      const float q = float(uint32_t(bits) & ((1u << BITS) - 1));
+      bits >>= BITS, have -= BITS;
+      p = __builtin_fmaf(bf16f(x[64 * g + k]), __builtin_fmaf(sg, q, bg), p);
+    }
+  }
+  return wave_sum_bfly(p);
+}
+
+// Row tiles of a block's range of the flat list [u, u1): the tile and its steps
+// at u, and u past them.
+struct Part {
+  int slot, p0, m, st0, st1;
+};
+
+__device__ __forceinline__ Part next_part(const StreamArgs& a, int n_st, int64_t& u, int64_t u1) {
+  typedef const __attribute__((address_space(4))) int32_t ConstI32;
+  const int tile = int(u / n_st);
+  Part t;
+  t.st0 = int(u - int64_t(tile) * n_st);
+  t.st1 = int(min(int64_t(n_st), t.st0 + (u1 - u)));
+  u += t.st1 - t.st0;
+  ConstI32* tl = (ConstI32*)(a.tiles + tile);
+  const int first = tl[1];
+  t.slot = tl[0];
+  t.p0 = tl[3] + first;
+  t.m = min(kStreamRows, tl[2] - first);
+  return t;
+}
+
+// The outputs of a block's range that came out infinite or NaN once more, with
+// plain products: (128 + q) x and 128 s sum(x) of an x above ~1e34 overflow
+// where (s q + b) x does not, and those of an infinity cancel to NaN.  (An
+// overflow on the way always reaches the output.  Scaling such rows in
+// registers cost the loops spills, a flag a tile 1-2% of a layer.)  Rows with a
+// NaN are left as they are.  Waves take 64 columns of a row at a time.
+template <int BITS, int NSL, int STEP_COLS, bool DUAL, bool F32>
+__device__ __forceinline__ void redo_range(const StreamArgs& a, int n_st, int64_t u, int64_t u1) {
+  using Out = std::conditional_t<F32, float, uint16_t>;
+  constexpr uint32_t kInf = F32 ? 0x7F800000u : 0x7F80u;
+  const int lane = threadIdx.x & 63;
+  const int groups = a.cols / 64;
+  const size_t row_bytes = size_t(a.cols) * BITS / 8;
+#pragma unroll 1
+  while (u < u1) {
+    const Part t = next_part(a, n_st, u, u1);
+    if (t.slot < 0) continue;
+    const uint8_t* slot = a.slab + size_t(t.slot) * size_t(a.expert_bytes);
+#pragma unroll 1
+    for (int p = t.p0; p < t.p0 + t.m; ++p) {
+      const int flat = a.order[p];
+      const uint16_t* x = a.act + size_t(DUAL ? flat / a.kk : p) * a.cols;
+      Out* out = static_cast<Out*>(a.out) + size_t(DUAL ? p : flat) * a.out_cols;
+      bool nan = false;
+      for (int k = lane; k < a.cols; k += 64) nan |= (x[k] & 0x7FFFu) > 0x7F80u;
+      if (__ballot(nan)) continue;
+      const int c1 = t.st1 * STEP_COLS;
+#pragma unroll 1
+      for (int c0 = t.st0 * STEP_COLS + int(threadIdx.x & ~63u); c0 < c1; c0 += 64 * NSL) {
+        const uint32_t v =
+            c0 + lane < c1
+                ? reinterpret_cast<const std::conditional_t<F32, uint32_t, uint16_t>*>(out)[c0 + lane]
+                : 0u;
+#pragma unroll 1
+        for (uint64_t odd = __ballot((v & kInf) == kInf); odd; odd &= odd - 1) {
+          const int c = c0 + __builtin_ctzll(odd);
+          auto dot = [&](const QProj& q) {
+            return plain_dot<BITS>(
+                reinterpret_cast<const uint32_t*>(slot + q.w + c * row_bytes),
+                reinterpret_cast<const uint16_t*>(slot + q.s) + size_t(c) * groups,
+                reinterpret_cast<const uint16_t*>(slot + q.b) + size_t(c) * groups, x, groups);
+          };
+          float y = dot(a.p0);
+          if constexpr (DUAL) y = silu_fast(y) * dot(a.p1);
+          if (lane) continue;
+          if constexpr (F32)
+            out[c] = y;
+          else
+            out[c] = f2bf(y);
+        }
+      }
+    }
+  }
+}
 
 template <int BITS, int G, int NSL, bool DUAL, bool F32>
 __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a) {
@@ -406,21 +517,19 @@ __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a)
   typedef const __attribute__((address_space(4))) int32_t ConstI32;
   __shared__ __attribute__((aligned(16))) float part[K::kLds];
   __shared__ int32_t s_row[2][kStreamRows];
+  __shared__ uint32_t s_odd;  // an output of this block is not finite
   const int n_st = a.out_cols / K::kStepCols;
   const int64_t total = int64_t(*(ConstI32*)a.n_tiles) * n_st;
+  const int64_t u0 = total * blockIdx.x / gridDim.x;
   const int64_t u1 = total * (blockIdx.x + 1) / gridDim.x;
-  int64_t u = total * blockIdx.x / gridDim.x;
   int buf = 0, par = 0;
-  while (u < u1) {
-    const int tile = int(u / n_st);
-    const int st0 = int(u - int64_t(tile) * n_st);
-    const int st1 = int(min(int64_t(n_st), st0 + (u1 - u)));
-    u += st1 - st0;
-    ConstI32* tl = (ConstI32*)(a.tiles + tile);
-    const int slot = tl[0], first = tl[1], cnt = tl[2], off = tl[3];
+  if (threadIdx.x == 0) s_odd = 0;  // seen by all from the first step's barrier
+  for (int64_t u = u0; u < u1;) {
+    const Part t = next_part(a, n_st, u, u1);
+    const int st0 = t.st0, st1 = t.st1, slot = t.slot;
     Seg sg;
-    sg.p0 = off + first;
-    sg.m = min(kStreamRows, cnt - first);
+    sg.p0 = t.p0;
+    sg.m = t.m;
     sg.slot = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(a.slab) + size_t(max(slot, 0)) * size_t(a.expert_bytes), 0,
         uint32_t(a.expert_bytes), 0x00027000);
@@ -442,14 +551,20 @@ __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a)
     }
     if constexpr (K::kMaxMT == 2) {
       if (sg.m > 16)
-        K::template run<2>(a, sg, 0, st0, st1, part, buf, s_row[par]);
+        K::template run<2>(a, sg, 0, st0, st1, part, buf, s_row[par], &s_odd);
       else
-        K::template run<1>(a, sg, 0, st0, st1, part, buf, s_row[par]);
+        K::template run<1>(a, sg, 0, st0, st1, part, buf, s_row[par], &s_odd);
     } else {
       for (int r0 = 0; r0 < sg.m; r0 += 16)
-        K::template run<1>(a, sg, r0, st0, st1, part, buf, s_row[par]);
+        K::template run<1>(a, sg, r0, st0, st1, part, buf, s_row[par], &s_odd);
     }
     par ^= 1;
+  }
+  block_lds_sync();
+  if (__builtin_amdgcn_readfirstlane(s_odd)) {
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's stores, then every wave's
+    __syncthreads();
+    redo_range<BITS, NSL, K::kStepCols, DUAL, F32>(a, n_st, u0, u1);
   }
 }
 

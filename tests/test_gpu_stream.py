@@ -129,6 +129,54 @@ def test_stream_components_in_arrays_of_their_own(bits, monkeypatch):
     slab.release()
 
 
+@pytest.mark.parametrize("n", [7, 75])
+@pytest.mark.parametrize("bits,hidden,inter", [(4, 1024, 512), (6, 1024, 512), (4, 7168, 512)])
+def test_stream_huge_activations(bits, hidden, inter, n, monkeypatch):
+    """(128 + q) x and 128 s sum(x) of a huge or infinite x leave fp32 where
+    (s q + b) x does not.  Finite rows: a 3e38 against weights of ~1e-20 stays
+    finite, within tests/util's tolerance.  Infinite ones: NaN and the two
+    infinities where float64 has them (weights of one sign: infinities; both
+    signs: NaN).  A NaN spoils its own row only, and every other row keeps its
+    bits."""
+    from pagedmoe_amd import kernels as K
+    from pagedmoe_amd._lib import geom
+    from pagedmoe_amd.slab import SlabStore
+    monkeypatch.setenv("PMOE_STREAM", "1")
+    g = geom(hidden, inter, bits)
+    table = torch.arange(2, dtype=torch.int32, device=DEV)
+    rng = np.random.default_rng(97)
+    ids = np.stack([rng.permutation(2) for _ in range(n)]).astype(np.int32)
+    for std, positive, values in ((1e-20, False, {1: 3e38, 5: -1e36}),
+                                  (0.02, True, {2: np.inf, 6: np.nan}),
+                                  (0.02, False, {0: np.inf, 3: np.nan, 4: -np.inf})):
+        slab = SlabStore(g, 2, DEV)
+        gen = torch.Generator(device=DEV).manual_seed(98)
+        for slot in range(2):
+            for proj, rows, cols in (("gate_proj", inter, hidden), ("up_proj", inter, hidden),
+                                     ("down_proj", hidden, inter)):
+                w = torch.randn((rows, cols), generator=gen, device=DEV) * std
+                slab.quantize_into(slot, proj, w.abs() if positive else w)
+        plain = rng.standard_normal((n, hidden)).astype(np.float32)
+        odd = plain.copy()
+        for row, v in values.items():
+            odd[row, 7 * row + 3] = v
+        bits_of = [O.bf16_round(a) for a in (plain, odd)]
+        base, y = (_run(K, g, slab, table, 2, xb, ids).float().cpu().numpy() for xb in bits_of)
+        rest = [i for i in range(n) if i not in values]
+        assert np.array_equal(base[rest].view(np.int32), y[rest].view(np.int32))
+        rows = sorted(values)
+        with np.errstate(all="ignore"):
+            ref = O.switch_glu_f64(bits_of[1][rows], ids[rows], [slot_to_expert(slab, e)
+                                                                 for e in range(2)])
+        for i, row in enumerate(rows):
+            if np.isfinite(values[row]):
+                check_close(y[row], ref[i], f"row of {values[row]}")
+            else:
+                for same in (np.isnan, np.isposinf, np.isneginf):
+                    assert np.array_equal(same(y[row]), same(ref[i])), (values[row], same)
+        slab.release()
+
+
 @pytest.mark.parametrize("bits,n", [(4, 2), (4, 12), (4, 13), (4, 17), (6, 50)])
 def test_stream_block_vs_oracle(bits, n, monkeypatch):
     """The whole block with a gated shared expert (its rows are every token:
