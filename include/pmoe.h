@@ -163,8 +163,11 @@ int pmoe_prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n
 
 /* 1 when the experts of n tokens with kk columns (shared: the last is a
  * shared expert's) run as streamed 16-column tiles: between the decode GEMV
- * (few rows an expert) and the prefill GEMMs (more than 32 rows an expert on
- * average); PMOE_STREAM=1 / 0 pins it where the shape is covered.  Slots whose
+ * (few rows an expert) and the prefill GEMMs (where they cover the call: dims
+ * that are multiples of 512, and more than 32 rows an expert on
+ * average, in layers of enough expert bytes).  PMOE_STREAM=1 / 0 pins it where
+ * the shape is covered: hidden and inter multiples of 128 from 384 to 7168
+ * (6-bit: to 4096; a wave holds its slice of a row in registers).  Slots whose
  * components do not all lie inside a stride below 2 GiB, on 4-byte offsets,
  * are not (nor is a slab that is not 4-byte aligned).  No reference
  * counterpart. */

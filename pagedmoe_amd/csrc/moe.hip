@@ -217,39 +217,48 @@ int check_route_cfg(const pmoe_route_cfg* rc) {
 
 // Whether the experts of n tokens with kk columns run as streamed MFMA tiles
 // (stream.hip) rather than as the decode GEMV or the prefill GEMMs.  Measured
-// us a layer, GEMV or prefill form / streamed, on either side of each line:
-//   upper end, 32 rows an expert on average (the 32-row prefill tiles'
-//     range): Qwen3-235B shapes 512 tokens 607 / 490, 700 tokens 538 / 594
-//     (128-row tiles); Qwen3-Next shapes 1000 tokens 422 / 399,
-//     1400 tokens 493 / 466.  Reductions
-//     above 4096 hold 16 rows a pass, not 32, and stop where the prefill GEMMs
-//     begin (DeepSeek-V3 shapes 600 tokens 25763 / 2734, 1000 tokens
-//     3183 / 3757).  Layers of hidden < 2048 keep the prefill GEMMs there,
-//     whose two tile heights give the same bits.
+// us a layer, GEMV or prefill form / streamed, on either side of each line
+// (hidden x inter x experts, top-8 unless said otherwise):
+//   upper end, where the prefill GEMMs cover the call: 32 rows an expert on
+//     average, the range of their 32-row tiles (4096x1536x128 512 tokens
+//     594 / 490, 700 tokens 538 / 594 at 128-row tiles).  Layers of hidden <
+//     2048 keep the GEMMs there (1024x512x128 512 tokens 73 / 90).  Reductions
+//     above 4096 hold 16 rows a pass, not 32, and stop where the GEMMs begin
+//     (5120x1536x160 top-6 600 tokens 777 / 828, 1200 tokens 864 / 1490).
+//     Dims that are no multiples of 512 have no GEMMs and no upper end
+//     (2048x768x128 600 tokens 1537 / 179, 4000 tokens 9666 / 678).
 //   lower end, where the GEMV's re-use of a weight row for the few rows of an
-//     expert runs out: 0.75 rows an expert for 4-bit (Qwen3-235B shapes 8
-//     tokens 129 / 148, 12 tokens 179 / 175, 20 tokens 273 / 226), a third for
-//     6-bit (Qwen3-Next shapes 8 tokens 69 / 88, 16 tokens 123 / 122, 24
-//     tokens 233 / 138), 16
-//     rows for reductions above 4096 (DeepSeek-V3 shapes 2 tokens 134 / 122,
-//     8 tokens 438 / 316); and 128 MiB of GEMV reads (rows x expert bytes), so
-//     that the extra launches pay (hidden 1024, 32 experts: 24 tokens 46 / 50,
-//     40 tokens 61 / 54).
+//     expert runs out: 0.75 rows an expert for 4-bit (4096x1536x128 8 tokens
+//     129 / 148, 12 tokens 179 / 175, 20 tokens 273 / 226), a third for 6-bit
+//     (2048x512x512 8 tokens 69 / 88, 16 tokens 123 / 122, 24 tokens
+//     233 / 138); and enough bytes that it reads more than once to pay for the
+//     extra launches, 100 MiB and 64 MiB (4-bit: 2048x768x128 12 tokens,
+//     72 MiB, 68 / 74, 15 tokens, 106 MiB, 78 / 69; 2048x512x128 16 tokens,
+//     79 MiB, 63 / 65, 24 tokens, 156 MiB, 81 / 74; 4096x1536x8 top-2 8 tokens,
+//     90 MiB, 42 / 53, 16 tokens, 243 MiB, 66 / 48; 6-bit: 2048x768x128
+//     8 tokens, 50 MiB, 66 / 76, 14 tokens, 138 MiB, 103 / 95; 2304x1152x64
+//     top-6 4 tokens, 25 MiB, 57 / 63, 8 tokens, 88 MiB, 92 / 79).  Reductions
+//     above 4096: 16 rows and 128 MiB of GEMV reads (7168x2048x384 and a
+//     shared expert 2 tokens 134 / 122, 8 tokens 438 / 316; 5120x1536x160 top-6
+//     2 tokens 63 / 64, 4 tokens 101 / 95).
 // PMOE_STREAM=1 / 0 pins the form where it covers the shape (read per call, so
-// the two can be compared).
+// the two can be compared); a pinned prefill tile height keeps the GEMMs.
 bool stream_wanted(const pmoe_geom* g, const uint8_t* slab, int n, int kk, int n_experts,
                    int n_ids) {
   if (!stream_covers(g, slab)) return false;
   const char* v = getenv("PMOE_STREAM");
   if (v && (v[0] == '0' || v[0] == '1')) return v[0] == '1';
-  const long rows = long(n) * kk;
+  const int64_t rows = int64_t(n) * kk, mib = 1 << 20;
   const bool wide = g->hidden > 4096 || g->inter > 4096;
+  const bool four = g->bits == 4;
   if (prefill_wanted(g, n, kk, n_ids) &&
-      (wide || g->hidden < 2048 || getenv("PMOE_PREFILL_SMALL")))
+      (wide || rows > 32L * n_experts || getenv("PMOE_PREFILL_SMALL") ||
+       g->hidden < 2048))
     return false;
-  if (rows > 32L * n_experts || rows * g->expert_bytes < (128L << 20)) return false;
-  if (wide) return rows >= 16;
-  return g->bits == 4 ? 4 * rows >= 3L * n_experts : 3 * rows >= n_experts;
+  if (wide) return rows >= 16 && rows * g->expert_bytes >= 128 * mib;
+  if (four ? 4 * rows < 3L * n_experts : 3 * rows < n_experts) return false;
+  const double distinct = n_experts * (1.0 - exp(-double(rows) / n_experts));  // of even routing
+  return (rows - distinct) * double(g->expert_bytes) >= double((four ? 100 : 64) * mib);
 }
 
 // Dispatch + the three projections (+ SwiGLU) for rows = n*kk flat rows.
@@ -405,9 +414,12 @@ int decode_block(const pmoe_geom* g, const pmoe_route_cfg* rc, const uint8_t* sl
   if (n > 1 && !getenv("PMOE_DECODE_FUSED") && stream_wanted(g, slab, n, kk, e, e + shared)) {
     // Up to 12 tokens the router launch's last block routes, one token a wave
     // and round; beyond, its rounds cost more than a routing launch with a wave
-    // for every token (us a layer, last block / launch: Qwen3-235B shapes 12
-    // tokens 180 / 183, 16 tokens 199 / 197, 29 tokens 272 / 264; Qwen3-Next
-    // shapes 23 tokens 144 / 134).
+    // for every token (us a layer, last block / launch: 7168x2048x384 with
+    // sigmoid scores 4 tokens 199 / 209, 8 tokens 309 / 315, 12 tokens 382 / 382,
+    // 24 tokens 871 / 859; 5120x1536x160 8 tokens 153 / 157, 12 tokens 197 / 200,
+    // 24 tokens 444 / 442; 3072x1536x64 8 to 16 tokens within 1, 24 tokens
+    // 130 / 125; 4096x1536x128 12 tokens 181 / 179, 29 tokens 274 / 266;
+    // 2048x512x512 23 tokens 147 / 137; 1024x512x32 64 tokens 57 / 46).
     constexpr int kRouteTailTokens = 12;
     int r;
     if (n <= kRouteTailTokens) {

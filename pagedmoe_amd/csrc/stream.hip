@@ -47,6 +47,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u32x3_a4 __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -79,26 +80,34 @@ struct WTile {
   static constexpr int kRegs = BITS == 4 ? 2 * G : 3 * G;
   using V = std::conditional_t<BITS == 4, u32x4, u32x3_a4>;
   static constexpr int kS4 = G / 8;               // scale words: vectors of 4,
-  static constexpr int kS3 = (G % 8) / 2 == 3;    // then one of 3
-  static_assert(kS4 * 8 + kS3 * 6 == G, "groups a slice: 8 i or 8 i + 6");
+  static constexpr int kSR = (G % 8) / 2;         // then one of the 0-3 left
+  static_assert(G % 2 == 0, "scales are read as whole words");
+  using R = std::conditional_t<kSR == 1, uint32_t,
+                               std::conditional_t<kSR == 2, u32x2_a4, u32x3_a4>>;
   V w[kV];
   u32x4_a4 s4[kS4 ? kS4 : 1], b4[kS4 ? kS4 : 1];
-  u32x3_a4 s3, b3;
+  R sr, br;
   __device__ __forceinline__ uint32_t word(int i) const {
     return BITS == 4 ? w[i >> 2][i & 3] : w[i / 3][i % 3];
   }
   __device__ __forceinline__ uint32_t s(int i) const {
-    return i < 4 * kS4 ? s4[i < 4 * kS4 ? i >> 2 : 0][i & 3] : s3[i - 4 * kS4];
+    return i < 4 * kS4 ? s4[i < 4 * kS4 ? i >> 2 : 0][i & 3] : rest(sr, i - 4 * kS4);
   }
   __device__ __forceinline__ uint32_t b(int i) const {
-    return i < 4 * kS4 ? b4[i < 4 * kS4 ? i >> 2 : 0][i & 3] : b3[i - 4 * kS4];
+    return i < 4 * kS4 ? b4[i < 4 * kS4 ? i >> 2 : 0][i & 3] : rest(br, i - 4 * kS4);
+  }
+  static __device__ __forceinline__ uint32_t rest(const R& r, int i) {
+    if constexpr (kSR == 1)
+      return r;
+    else
+      return r[i];
   }
   // Opaque to the optimiser: without this, unpacking moves to the end of the
   // loop trip that loaded the words and waits for them there.
   __device__ __forceinline__ void pin() {
 #pragma unroll
     for (int i = 0; i < kS4; ++i) asm volatile("" : "+v"(s4[i]), "+v"(b4[i]));
-    if constexpr (kS3) asm volatile("" : "+v"(s3), "+v"(b3));
+    if constexpr (kSR != 0) asm volatile("" : "+v"(sr), "+v"(br));
 #pragma unroll
     for (int i = 0; i < kV; ++i) asm volatile("" : "+v"(w[i]));
   }
@@ -128,9 +137,15 @@ __device__ __forceinline__ void load_tile(WTile<BITS, G>& t, __amdgpu_buffer_rsr
     t.s4[i] = __builtin_amdgcn_raw_buffer_load_b128(slot, s_off + 16 * i, s, 0);
     t.b4[i] = __builtin_amdgcn_raw_buffer_load_b128(slot, s_off + 16 * i, b, 0);
   }
-  if constexpr (T::kS3) {
-    t.s3 = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, s, 0);
-    t.b3 = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, b, 0);
+  if constexpr (T::kSR == 3) {
+    t.sr = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, s, 0);
+    t.br = __builtin_amdgcn_raw_buffer_load_b96(slot, s_off + 16 * T::kS4, b, 0);
+  } else if constexpr (T::kSR == 2) {
+    t.sr = __builtin_amdgcn_raw_buffer_load_b64(slot, s_off + 16 * T::kS4, s, 0);
+    t.br = __builtin_amdgcn_raw_buffer_load_b64(slot, s_off + 16 * T::kS4, b, 0);
+  } else if constexpr (T::kSR == 1) {
+    t.sr = __builtin_amdgcn_raw_buffer_load_b32(slot, s_off + 16 * T::kS4, s, 0);
+    t.br = __builtin_amdgcn_raw_buffer_load_b32(slot, s_off + 16 * T::kS4, b, 0);
   }
 }
 
@@ -150,8 +165,9 @@ struct XTile {
   float sum[(G + 3) / 4];
 };
 
+// The first `repeat` groups are the slice before's too and count as zero here.
 template <int BITS, int G>
-__device__ __forceinline__ void load_x(XTile<G>& x, const uint16_t* src, int kq) {
+__device__ __forceinline__ void load_x(XTile<G>& x, const uint16_t* src, int kq, int repeat) {
   constexpr uint32_t kOnes = 0x3F803F80u;
 #pragma unroll
   for (int g = 0; g < G; ++g)
@@ -162,16 +178,19 @@ __device__ __forceinline__ void load_x(XTile<G>& x, const uint16_t* src, int kq)
   for (int q = 0; q < (G + 3) / 4; ++q) x.sum[q] = 0.0f;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
+    const uint32_t keep = g < repeat ? 0u : ~0u;
     float s = 0.0f;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const u32x4 d = x.a[g][c];
+      const u32x4 d = x.a[g][c] & keep;
       s = dot2(d[3], kOnes, dot2(d[2], kOnes, dot2(d[1], kOnes, dot2(d[0], kOnes, s))));
       if constexpr (BITS == 4)  // pairs (x_i, x_{i+4}), as nib_pair unpacks
         x.a[g][c] = u32x4{__builtin_amdgcn_perm(d[2], d[0], 0x05040100u),
                           __builtin_amdgcn_perm(d[2], d[0], 0x07060302u),
                           __builtin_amdgcn_perm(d[3], d[1], 0x05040100u),
                           __builtin_amdgcn_perm(d[3], d[1], 0x07060302u)};
+      else
+        x.a[g][c] = d;
     }
     s = s + xor_lane<32>(s);
     s = s + xor_lane<16>(s);
@@ -308,6 +327,9 @@ struct StreamKernel {
     const int m = sg.m - r0;
     const uint32_t row_bytes = uint32_t(a.cols) * BITS / 8;
     const uint32_t groups = uint32_t(a.cols) / 64;
+    // first group of the slice: the last slices of an uneven cut move back to
+    // end with the row
+    const int g0 = min(slice * G, int(groups) - G);
     const uint32_t w_off = row * row_bytes + kq * (BITS == 4 ? 16 : 12);
     const uint32_t s_off = row * groups * 2;
     WTile<BITS, G> W[E];
@@ -315,9 +337,9 @@ struct StreamKernel {
     auto load = [&](int e, int t0, int step) {
       const QProj& q = DUAL && (e & 1) ? a.p1 : a.p0;
       const uint32_t r = (step * (kStepCols / kCols) + (DUAL ? (t0 + e) >> 1 : t0 + e)) * kCols;
-      const uint32_t g = slice * (G * 2) + r * groups * 2;
+      const uint32_t g = g0 * 2 + r * groups * 2;
       load_tile<BITS, G>(W[e], sg.slot, w_off,
-                         uint32_t(q.w) + slice * (G * 64 * BITS / 8) + r * row_bytes, s_off,
+                         uint32_t(q.w) + g0 * (64 * BITS / 8) + r * row_bytes, s_off,
                          uint32_t(q.s) + g, uint32_t(q.b) + g);
     };
     int ar[MT];
@@ -332,8 +354,8 @@ struct StreamKernel {
     XTile<G> x[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      load_x<BITS, G>(x[mt], a.act + size_t(ar[mt]) * a.cols + slice * (G * 64) +
-                                 quarter_k<BITS>(kq), kq);
+      load_x<BITS, G>(x[mt], a.act + size_t(ar[mt]) * a.cols + g0 * 64 + quarter_k<BITS>(kq), kq,
+                      slice * G - g0);
     // Everything so far has arrived (the activations, requested last, are
     // needed at once): with nothing pending on entry, the compiler's wait
     // counts at the loop head are those of the steady state.  Left pending
@@ -568,21 +590,23 @@ __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a)
   }
 }
 
-// Slices of a reduction of `cols` values: {groups a slice, slices}, or zeros.
+// Slices of a reduction of `cols` values: {groups a slice, slices}, or zeros
+// where there is no cut.  The fewest waves whose x fits next to the ring at 32
+// rows (6 or 8 groups); beyond 64 groups 8 waves of 10, 12 or 14, at 16 rows a
+// pass.  Scales and biases are read as words, two groups each, so the count
+// has to be even; and a row is at least a slice.  An uneven cut reads the
+// groups its last slices share from L2 and multiplies them by zero: at most
+// 1.5 times the arithmetic (the first counts of 4 and 8 waves, 18 and 34).
 struct Cut {
   int g, nsl;
 };
 
 Cut stream_cut(int cols) {
-  switch (cols) {
-    case 512: return {8, 1};
-    case 1024: return {8, 2};
-    case 1536: return {6, 4};
-    case 2048: return {8, 4};
-    case 4096: return {8, 8};
-    case 7168: return {14, 8};
-    default: return {0, 0};
-  }
+  const int n = cols / 64;
+  if (cols % 128 || n < 6 || n > 112) return {0, 0};
+  for (int nsl = 1; nsl <= 8; nsl *= 2)
+    if (n <= 8 * nsl) return {n <= 6 * nsl ? 6 : 8, nsl};
+  return {n <= 80 ? 10 : n <= 96 ? 12 : 14, 8};
 }
 
 // Blocks: every CU filled with 8 waves (two a SIMD).
@@ -597,12 +621,17 @@ int launch_stream(const StreamArgs& a, hipStream_t st) {
     PMOE_LAUNCH_CHECK("stream_kernel");                                                \
     return PMOE_OK;                                                                    \
   }
+  PMOE_CASE(6, 1)
   PMOE_CASE(8, 1)
+  PMOE_CASE(6, 2)
   PMOE_CASE(8, 2)
   PMOE_CASE(6, 4)
   PMOE_CASE(8, 4)
+  PMOE_CASE(6, 8)
   PMOE_CASE(8, 8)
   if constexpr (BITS == 4) {
+    PMOE_CASE(10, 8)
+    PMOE_CASE(12, 8)
     PMOE_CASE(14, 8)
   }
 #undef PMOE_CASE

@@ -48,6 +48,9 @@ def _run(K, g, slab, table, n_experts, xb, ids):
 @pytest.mark.parametrize("hidden,inter,bits", [
     (1024, 512, 4), (1024, 512, 6), (2048, 512, 6), (2048, 1536, 4), (4096, 1536, 4),
     (4096, 1024, 6), (1536, 2048, 6), (7168, 2048, 4),
+    # uneven cuts: last slices that overlap the one before, or repeat it whole
+    (384, 640, 4), (384, 640, 6), (1408, 896, 4), (1408, 896, 6), (2560, 1152, 4),
+    (2560, 1152, 6), (3072, 768, 6), (5120, 768, 4), (5376, 384, 4), (6400, 2304, 4),
 ])
 def test_stream_seam_vs_oracle(hidden, inter, bits, monkeypatch):
     """Rows per expert 1, 15, 16, 17, 31, 32, 33, 70 and one absent expert;

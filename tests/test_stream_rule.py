@@ -13,7 +13,19 @@ import pytest
     (2048, 512, 6, 512, 11, {15: 0, 16: 1, 1489: 1, 1490: 0}),
     (7168, 2048, 4, 384, 9, {1: 0, 2: 1, 684: 1, 685: 0}),
     (1024, 512, 4, 32, 4, {37: 0, 38: 1, 255: 1, 256: 0}),
-    (1024, 768, 4, 32, 4, {64: 0}),
+    # dims without prefill GEMMs (no multiples of 512) have no upper end
+    (2048, 768, 4, 128, 8, {12: 0, 16: 1, 600: 1, 16384: 1}),
+    (2304, 1152, 6, 64, 6, {4: 0, 8: 1, 4096: 1}),
+    (384, 640, 4, 64, 4, {16: 0, 4096: 1}),
+    # 128-row tiles' layers below 1024 rows are the GEMV's otherwise
+    (6144, 2560, 4, 16, 2, {4: 0, 8: 1, 511: 1, 512: 0}),
+    (5120, 1536, 4, 160, 6, {2: 0, 4: 1, 426: 1, 427: 0}),
+    # no cut: odd group counts, rows below six groups, 6-bit rows above 4096
+    (2880, 2880, 4, 32, 4, {64: 0, 4096: 0}),
+    (1024, 704, 4, 32, 4, {64: 0}),
+    (1024, 256, 4, 32, 4, {64: 0}),
+    (7168, 2048, 6, 64, 8, {64: 0}),
+    (8192, 1024, 4, 16, 2, {64: 0}),
 ])
 def test_stream_rule(hidden, inter, bits, e, kk, form, monkeypatch):
     for v in ("PMOE_STREAM", "PMOE_PREFILL_SMALL"):
