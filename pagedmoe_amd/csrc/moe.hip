@@ -221,8 +221,14 @@ int check_route_cfg(const pmoe_route_cfg* rc) {
 // (hidden x inter x experts, top-8 unless said otherwise):
 //   upper end, where the prefill GEMMs cover the call: 32 rows an expert on
 //     average, the range of their 32-row tiles (4096x1536x128 512 tokens
-//     594 / 490, 700 tokens 538 / 594 at 128-row tiles).  Layers of hidden <
-//     2048 keep the GEMMs there (1024x512x128 512 tokens 73 / 90).  Reductions
+//     594 / 490, 700 tokens 538 / 594 at 128-row tiles), and layers whose
+//     experts together are long enough a stream: 256 MiB at 4 bits
+//     (16, 25 and 32 rows an expert: 2048x512x128, 216 MiB, 93 / 87, 109 / 110
+//     and 111 / 125; 2560x512x128, 270 MiB, 119 / 112, 140 / 130 and 150 / 152;
+//     2048x512x256, 432 MiB, 176 / 150, 194 / 175 and 217 / 204), 768 MiB at 6
+//     (2048x512x128, 312 MiB, 114 / 114, 136 / 142 and 144 / 159; 4096x512x128,
+//     624 MiB, 207 / 201, 247 / 234 and 261 / 272; 2048x512x512, 1.2 GiB, top-10
+//     and a shared expert, 432 / 390, 445 / 421 and 504 / 497).  Reductions
 //     above 4096 hold 16 rows a pass, not 32, and stop where the GEMMs begin
 //     (5120x1536x160 top-6 600 tokens 777 / 828, 1200 tokens 864 / 1490).
 //     Dims that are no multiples of 512 have no GEMMs and no upper end
@@ -253,7 +259,7 @@ bool stream_wanted(const pmoe_geom* g, const uint8_t* slab, int n, int kk, int n
   const bool four = g->bits == 4;
   if (prefill_wanted(g, n, kk, n_ids) &&
       (wide || rows > 32L * n_experts || getenv("PMOE_PREFILL_SMALL") ||
-       g->hidden < 2048))
+       n_experts * g->expert_bytes < (four ? 256 : 768) * mib))
     return false;
   if (wide) return rows >= 16 && rows * g->expert_bytes >= 128 * mib;
   if (four ? 4 * rows < 3L * n_experts : 3 * rows < n_experts) return false;

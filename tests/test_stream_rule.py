@@ -19,6 +19,11 @@ import pytest
     (384, 640, 4, 64, 4, {16: 0, 4096: 1}),
     # 128-row tiles' layers below 1024 rows are the GEMV's otherwise
     (6144, 2560, 4, 16, 2, {4: 0, 8: 1, 511: 1, 512: 0}),
+    # the prefill range, by the layer's bytes: 216, 270, 312 and 1224 MiB
+    (2048, 512, 4, 128, 8, {255: 1, 257: 0, 512: 0}),
+    (2560, 512, 4, 128, 8, {255: 1, 257: 1, 512: 1, 513: 0}),
+    (2048, 512, 6, 128, 8, {255: 1, 257: 0}),
+    (2048, 512, 6, 512, 10, {820: 1, 1638: 1, 1639: 0}),
     (5120, 1536, 4, 160, 6, {2: 0, 4: 1, 426: 1, 427: 0}),
     # no cut: odd group counts, rows below six groups, 6-bit rows above 4096
     (2880, 2880, 4, 32, 4, {64: 0, 4096: 0}),
