@@ -17,8 +17,7 @@ namespace pmoe {
 
 int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                     const int32_t* order, const int4* tiles, const int32_t* n_tiles, int tile_m,
-                    int max_tiles, int n_experts, uint16_t* h, void* y, int y_f32,
-                    hipStream_t st);
+                    int max_tiles, int n_experts, uint16_t* h, uint16_t* y, hipStream_t st);
 int prefill_tile_rows(int n, int kk, int n_experts);
 int prefill_min_tile_rows();
 bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids);
@@ -284,10 +283,13 @@ int run_experts(const pmoe_geom* g, const uint8_t* slab, const int32_t* table, i
   if (rc) return rc;
   if (stream)
     return stream_experts(g, slab, x, n, kk, w.order, w.tiles, w.n_tiles, w.h, y, y_f32, st);
-  if (prefill)
+  if (prefill) {
+    // fp32 rows are the streamed block path's alone (decode_block)
+    PMOE_REQUIRE(!y_f32, "prefill: outputs are bf16");
     return prefill_experts(g, slab, x, n, kk, w.order, w.tiles, w.n_tiles, tm,
-                           std::min(rows / tm + n_ids + 1, w.max_tiles), n_experts, w.h, y,
-                           y_f32, st);
+                           std::min(rows / tm + n_ids + 1, w.max_tiles), n_experts, w.h,
+                           static_cast<uint16_t*>(y), st);
+  }
   const int max_experts = rows < n_ids ? rows : n_ids;
   GemvArgs a{};
   a.slab = slab;

@@ -62,7 +62,6 @@ struct PrefillArgs {
   int64_t w1, s1, b1;    // and of the second (up for gate/up; = first for down)
   int out_cols;          // inter (h) or hidden (y)
   void* out;
-  int out_f32;
   int out_vec;           // out is 16-byte aligned: bf16 rows may go out as 16-byte pieces
 };
 
@@ -841,10 +840,7 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
   if (ti.slot < 0) {  // not resident: exact zero rows (streaming.py:715-719)
     for (int row = h; row < ti.m; row += 2) {
       const size_t o = size_t(a.order[ti.p0 + row]) * a.out_cols;
-      if (a.out_f32)
-        static_cast<float*>(a.out)[o + col] = 0.0f;
-      else
-        static_cast<uint16_t*>(a.out)[o + col] = 0;
+      static_cast<uint16_t*>(a.out)[o + col] = 0;
     }
     return;
   }
@@ -877,7 +873,7 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
   constexpr int kEp = kDnCols + 8;
   constexpr int kPieces = kDnCols / 8;
   constexpr bool kStaged = 32 * MB * kEp * 2 <= down_lds_bytes<BITS, MB>();
-  if (!kStaged || a.out_f32 || !a.out_vec) {
+  if (!kStaged || !a.out_vec) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
@@ -885,10 +881,7 @@ __global__ __launch_bounds__(kThreads, MB < kMB ? 4 : 1) void down_mfma_kernel(c
         const int row = mb * 32 + acc_row(r, h);
         if (row < ti.m) {
           const size_t o = size_t(s_ord[row]) * a.out_cols;
-          if (a.out_f32)
-            static_cast<float*>(a.out)[o + col] = acc[mb][r];
-          else
-            static_cast<uint16_t*>(a.out)[o + col] = f2bf(acc[mb][r]);
+          static_cast<uint16_t*>(a.out)[o + col] = f2bf(acc[mb][r]);
         }
       }
     }
@@ -1130,7 +1123,8 @@ __device__ __forceinline__ void gemm_tile_wide(int n_groups, const uint8_t* act,
           // block after next.  4-bit: set 1's words are one 16-byte read, and
           // step 0 dequantized from it.  6-bit: three reads, and step 0 uses
           // the first alone, so the others are waited for here (with step 1's
-          // fragments, which its MFMAs need at once).
+          // fragments, which its MFMAs need at once; waiting for the words
+          // alone was no faster).
           if (BITS == 6) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             load_w(j + 3, buf);
@@ -1250,10 +1244,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
   if (ti.slot < 0) {  // not resident: exact zero rows (streaming.py:715-719)
     for (int row = 0; row < ti.m; ++row) {
       const size_t o = size_t(a.order[ti.p0 + row]) * a.out_cols + cb * kWideDnCols + threadIdx.x;
-      if (a.out_f32)
-        static_cast<float*>(a.out)[o] = 0.0f;
-      else
-        static_cast<uint16_t*>(a.out)[o] = 0;
+      static_cast<uint16_t*>(a.out)[o] = 0;
     }
     return;
   }
@@ -1274,7 +1265,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
   gemm_wide_any<BITS>(nmb, groups, reinterpret_cast<const uint8_t*>(a.act), nullptr, 1, a.cols, ti.p0,
                 ti.m, wr, lds, acc);
   const int h = lane >> 5;
-  if (a.out_f32 || !a.out_vec) {
+  if (!a.out_vec) {
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -1284,10 +1275,7 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const PrefillArg
           const int row = mb * 32 + acc_row(r, h);
           if (row < ti.m) {
             const size_t o = size_t(s_ord[row]) * a.out_cols + col0 + 32 * c + (lane & 31);
-            if (a.out_f32)
-              static_cast<float*>(a.out)[o] = acc[c][mb][r];
-            else
-              static_cast<uint16_t*>(a.out)[o] = f2bf(acc[c][mb][r]);
+            static_cast<uint16_t*>(a.out)[o] = f2bf(acc[c][mb][r]);
           }
         }
     return;
@@ -1386,8 +1374,7 @@ bool prefill_wide(const pmoe_geom* g, const void* slab, const void* x, int n, in
 
 int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, int n, int kk,
                     const int32_t* order, const int4* tiles, const int32_t* n_tiles, int tile_m,
-                    int max_tiles, int n_experts, uint16_t* h, void* y, int y_f32,
-                    hipStream_t st) {
+                    int max_tiles, int n_experts, uint16_t* h, uint16_t* y, hipStream_t st) {
   PMOE_REQUIRE(tile_m == 32 || tile_m == kTileM, "prefill: tile height must be 32 or 128");
   PMOE_REQUIRE(g->inter % 512 == 0 && g->hidden % 512 == 0,
                "prefill: hidden and inter must be multiples of 512");
@@ -1417,7 +1404,6 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
   a.b1 = g->off[PMOE_UP_B];
   a.out_cols = g->inter;
   a.out = h;
-  a.out_f32 = 0;
   {
     const int items = g->inter / kGuCols * max_tiles;
     dim3 grid((items + 7) / 8 * 8);  // a multiple of 8: xcd_work deals items per XCD
@@ -1446,7 +1432,6 @@ int prefill_experts(const pmoe_geom* g, const uint8_t* slab, const uint16_t* x, 
   a.b0 = a.b1 = g->off[PMOE_DOWN_B];
   a.out_cols = g->hidden;
   a.out = y;
-  a.out_f32 = y_f32;
   a.out_vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
   {
     const int items = g->hidden / kDnCols * max_tiles;
