@@ -29,7 +29,7 @@ COUNTS = [300, 129, 128, 127, 97, 96, 1, 31, 32, 33, 64, 65, 90]
 
 @pytest.mark.parametrize("hidden,inter,bits", [(1024, 512, 4), (2048, 1536, 4), (512, 1024, 4),
                                                (4096, 512, 4), (1024, 512, 6), (2048, 1536, 6),
-                                               (4096, 1024, 6)])
+                                               (4096, 1024, 6), (7168, 2048, 4), (1024, 2048, 6)])
 def test_wide_matches_narrow_and_oracle(hidden, inter, bits, monkeypatch):
     from pagedmoe_amd import kernels as K
     monkeypatch.setenv("PMOE_STREAM", "0")
@@ -131,6 +131,7 @@ def test_wide_block_in_a_graph(monkeypatch):
     x = bits_to_bf16_tensor(O.bf16_round(rng.standard_normal((520, 1024), dtype=np.float32)), DEV)
     table = torch.arange(8, dtype=torch.int32, device=DEV)
     rc = K.route_cfg("softmax", 8, 2)
+    assert _wide(g, slab, x, 520, 2, 8) == 1
     eager = K.moe_block(g, rc, slab.buf, table, gw, x)[0].clone()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):

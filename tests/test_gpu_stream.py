@@ -40,6 +40,12 @@ def _ids(counts, k, rng, n):
     return ids
 
 
+def _streamed(g, n, kk, e, shared=0):
+    """The rule that the call itself asks."""
+    from pagedmoe_amd._lib import lib
+    return lib().pmoe_stream_wanted(ctypes.byref(g), n, kk, e, shared) == 1
+
+
 def _run(K, g, slab, table, n_experts, xb, ids):
     return K.switch_glu(g, slab.buf, table, n_experts, bits_to_bf16_tensor(xb, DEV),
                         torch.from_numpy(ids).to(DEV))
@@ -68,7 +74,8 @@ def test_stream_seam_vs_oracle(hidden, inter, bits, monkeypatch):
     table[8] = -1
     with KernelTimer() as kt:
         y = _run(K, g, slab, table, e, xb, ids).float().cpu().numpy()
-    assert "prefill_gateup" in kt.result and "gateup" not in kt.result, kt.result
+    assert _streamed(g, n, k, e) and "prefill_gateup" in kt.result, kt.result
+    assert "qgemv_gateup" not in kt.result, kt.result
     gone = (ids < 0) | (ids == 8)
     assert (y[gone] == 0).all()
     ref = O.switch_glu_f64(xb, np.where(gone, 0, ids), experts)
@@ -178,6 +185,52 @@ def test_stream_huge_activations(bits, hidden, inter, n, monkeypatch):
                 for same in (np.isnan, np.isposinf, np.isneginf):
                     assert np.array_equal(same(y[row]), same(ref[i])), (values[row], same)
         slab.release()
+
+
+# the block path's workspace starts with this synchronisation header (pmoe.h)
+HEADER = 1_352_960
+
+
+@pytest.mark.parametrize("n", [2, 12, 13, 28])
+@pytest.mark.parametrize("shape", [(1024, 512, 4), (1024, 512, 6), (2048, 768, 4)])
+@pytest.mark.parametrize("form", ["softmax", "softmax-shared", "sigmoid", "sigmoid-shared"])
+def test_stream_block_forms(form, shape, n, monkeypatch):
+    """Routing on both sides of its 12-token line (the router launch's last
+    block, a launch of its own), softmax and grouped sigmoid, with an ungated
+    shared expert and without one, and the busiest expert absent: its rows are
+    written as fp32 zeros, over scratch left full of NaN."""
+    from pagedmoe_amd import kernels as K
+    monkeypatch.setenv("PMOE_STREAM", "1")
+    hidden, inter, bits = shape
+    scoring, shared = form.split("-")[0], int(form.endswith("shared"))
+    e, k = 32, 6
+    sig = dict(scoring="sigmoid", n_group=8, topk_group=4, routed_scale=2.5)
+    spec = O.LayerSpec(hidden, e, inter, k, bits=bits, shared=shared,
+                       **(sig if scoring == "sigmoid" else {}))
+    g, slab, experts = _setup(hidden, inter, bits, e + shared, 101)
+    rng = np.random.default_rng(102 + n)
+    gw = O.bf16_round(rng.standard_normal((e, hidden), dtype=np.float32) * np.float32(0.02))
+    bias = rng.standard_normal(e, dtype=np.float32) * np.float32(0.05)
+    xb = O.bf16_round(rng.standard_normal((n, hidden), dtype=np.float32))
+    ref_i, ref_w, y, _ = O.moe_layer_f64(spec, xb, gw, experts, bias=bias)
+    gone = int(np.bincount(ref_i.reshape(-1)).argmax())
+    y[ref_i == gone] = 0.0
+    ref = O.combine_f64(y, ref_w,
+                        O.expert_ffn_f64(O.bf16_to_f32(xb), experts[e]) if shared else None)
+    table = torch.arange(e, dtype=torch.int32, device=DEV)
+    table[gone] = -1
+    rc = (K.route_cfg("sigmoid", e, k, True, 8, 4, 2.5) if scoring == "sigmoid"
+          else K.route_cfg("softmax", e, k))
+    x = bits_to_bf16_tensor(xb, DEV)
+    assert _streamed(g, n, k + shared, e, shared)
+    K.moe_workspace(g, n, k, shared, e, x.device)[HEADER:].fill_(255)
+    out, gi, gwt = K.moe_block(g, rc, slab.buf, table, bits_to_bf16_tensor(gw, DEV), x,
+                               score_bias=torch.from_numpy(bias).to(DEV)
+                               if scoring == "sigmoid" else None,
+                               shared_slot=e if shared else -1)
+    assert np.array_equal(gi.cpu().numpy(), ref_i) and np.array_equal(gwt.cpu().numpy(), ref_w)
+    check_close(out.float().cpu().numpy(), ref, f"{form} n={n}")
+    slab.release()
 
 
 @pytest.mark.parametrize("bits,n", [(4, 2), (4, 12), (4, 13), (4, 17), (6, 50)])
