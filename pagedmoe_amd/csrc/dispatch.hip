@@ -66,10 +66,11 @@ __device__ __forceinline__ int wave_rank(int my_e, int rows, const int* s_e, int
 
 // Rank of each thread's row among the earlier rows of its block with the same
 // expert, and the block's rows per expert (rows: how many the block has).
-// s_e[] holds the block's ids (-1: none, also past the rows; 16-byte aligned), s_wc[e * NW + w] receives wave
-// w's rows of expert e as a byte (at most 64) and must be zero.  A lane
-// compares its id with its wave's (wave_rank: broadcast reads), and the waves'
-// counts of an expert are read as one word or quad.  (One scan over all
+// s_e[] holds the block's ids (-1: none, also past the rows; 16-byte
+// aligned), s_wc[e * NW + w] receives wave w's rows of expert e as a byte (at
+// most 64) and must be zero.  A lane compares its id with its wave's
+// (wave_rank: broadcast reads), and the waves' counts of an expert are read as
+// one word or quad.  (One scan over all
 // earlier rows, up to 1,023 dependent steps, made an 800-row dispatch 16.0 us
 // (rocprof) against 8.1 now, and the 256-row counting blocks 6.2 against 4.9;
 // up to 64 rows one wave's ranks are all there is.)

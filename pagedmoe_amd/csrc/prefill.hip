@@ -1342,8 +1342,8 @@ bool prefill_wanted(const pmoe_geom* g, int n, int kk, int n_ids) {
 // 32 experts 1400 tokens 67 / 78, 2000 tokens 98 / 81, 16000 tokens 411 / 366;
 // Qwen3-235B shapes 520 tokens 491 / 492, 2048 tokens 1044 / 967, 8192 tokens
 // 3346 / 2851; DeepSeek-V3 shapes 2048 tokens 3717 / 3372; Qwen3-Next shapes
-// (6-bit) 1500 tokens 672 / 574, 5000 tokens 1004 / 883, 16000 tokens 2760 /
-// 2308.  Tiles are estimated as full ones plus half of one an expert.
+// (6-bit) 1500 tokens 666 / 587, 5000 tokens 1022 / 920, 16000 tokens 2804 /
+// 2391.  Tiles are estimated as full ones plus half of one an expert.
 // PMOE_PREFILL_WIDE=1 / 0 pins either (same outputs) where the wide form can run.
 //
 // It moves 16 bytes a lane from the activations and the weights straight into

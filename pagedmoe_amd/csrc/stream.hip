@@ -7,8 +7,8 @@
 // These sizes are bound by the weight stream, so the kernel is built around
 // it:
 //
-//   * The reduction is cut into NSL slices of G quantization groups, one
-//     wave each; a wave keeps its slice of the tile's 16 or 32 activation
+//   * The reduction is cut into NSL slices of G quantization groups
+//     (stream_cut), one wave each; a wave keeps its slice of the tile's 16 or 32 activation
 //     rows in registers as MFMA operands for as long as the tile lasts, and
 //     its inner loop only loads weights: tiles of 16 weight rows, a ring of
 //     them in flight, read as 16-byte (4-bit) or 12-byte (6-bit) pieces,
@@ -22,7 +22,7 @@
 //     tiles (double buffered, one LDS-only barrier, loads stay in flight
 //     across it).  With one or two tiles a step, 16 columns stored at a time
 //     and 64-bit vector addresses, Qwen3-Next shapes took 169 us a layer at
-//     24 tokens and 415 at 1000, against 138 and 399.
+//     24 tokens and 415 at 1000, against 138 and 405.
 //   * Work is the flat list (row tile, step), cut into equal contiguous
 //     ranges, one per resident block: every block streams the same number of
 //     bytes whatever the expert loads are.
@@ -31,7 +31,8 @@
 // -> 186 us (4.9 TB/s of weights), down 395 -> 103 us (4.4 TB/s) against the
 // GEMV, which repeats its dot products for every row of an expert; the same
 // loads without arithmetic, reduction and stores take 160 and 82 us.  8 waves
-// a CU at 256 registers: x takes 128 of them at 32 rows.
+// a CU at 256 registers: x takes 128 of them at 32 rows.  Only the 14-group
+// slices spill, around the weight loop, not in it.
 #include <algorithm>
 #include <type_traits>
 

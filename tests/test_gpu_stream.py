@@ -187,6 +187,31 @@ def test_stream_huge_activations(bits, hidden, inter, n, monkeypatch):
         slab.release()
 
 
+@pytest.mark.parametrize("n", [12, 13])
+def test_stream_block_huge_activations(n, monkeypatch):
+    """The block path's fp32 rows of a 3e38 against weights of ~1e-20."""
+    from pagedmoe_amd import kernels as K
+    from pagedmoe_amd._lib import geom
+    from pagedmoe_amd.slab import SlabStore
+    monkeypatch.setenv("PMOE_STREAM", "1")
+    g = geom(1024, 512, 4)
+    slab = SlabStore(g, 2, DEV)
+    fill_slab_gpu(slab, range(2), seed=103, std=1e-20)
+    xb = np.random.default_rng(104).standard_normal((n, 1024)).astype(np.float32)
+    xb[4, 100] = 3e38
+    xb = O.bf16_round(xb)
+    gate = torch.zeros((2, 1024), dtype=torch.bfloat16, device=DEV)
+    out, ids, w = K.moe_block(g, K.route_cfg("softmax", 2, 2), slab.buf,
+                              torch.arange(2, dtype=torch.int32, device=DEV), gate,
+                              bits_to_bf16_tensor(xb, DEV))
+    ids, w = ids.cpu().numpy(), w.cpu().numpy()
+    assert (w == 0.5).all()
+    ref = O.combine_f64(O.switch_glu_f64(xb[4:5], ids[4:5], [slot_to_expert(slab, e)
+                                                            for e in range(2)]), w[4:5])
+    check_close(out[4:5].float().cpu().numpy(), ref, "huge row of a block")
+    slab.release()
+
+
 # the block path's workspace starts with this synchronisation header (pmoe.h)
 HEADER = 1_352_960
 
