@@ -597,7 +597,7 @@ __global__ __launch_bounds__(64 * NSL, 2) void stream_kernel(const StreamArgs a)
 // pass.  Scales and biases are read as words, two groups each, so the count
 // has to be even; and a row is at least a slice.  An uneven cut reads the
 // groups its last slices share from L2 and multiplies them by zero: at most
-// 1.5 times the arithmetic (the first counts of 4 and 8 waves, 18 and 34).
+// 1.4 times the arithmetic (34 groups, the first count of 8 waves).
 struct Cut {
   int g, nsl;
 };

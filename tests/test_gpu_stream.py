@@ -206,8 +206,9 @@ def test_stream_block_huge_activations(n, monkeypatch):
                               bits_to_bf16_tensor(xb, DEV))
     ids, w = ids.cpu().numpy(), w.cpu().numpy()
     assert (w == 0.5).all()
-    ref = O.combine_f64(O.switch_glu_f64(xb[4:5], ids[4:5], [slot_to_expert(slab, e)
-                                                            for e in range(2)]), w[4:5])
+    with np.errstate(over="ignore"):  # exp of a hugely negative gate
+        ref = O.combine_f64(O.switch_glu_f64(xb[4:5], ids[4:5], [slot_to_expert(slab, e)
+                                                                for e in range(2)]), w[4:5])
     check_close(out[4:5].float().cpu().numpy(), ref, "huge row of a block")
     slab.release()
 
